@@ -357,10 +357,16 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_backward
   p.stream = c10::hip::getCurrentHIPStream(Q.device().index()).stream();
   torch::Tensor bits;  // lives until the launches are enqueued (stream-ordered reuse)
   if (attn_mask.has_value()) bits = pack_mask(*attn_mask, Q, K.size(2), p);
-  const int64_t ws = fa_sm75_backward_workspace_size(&p);
+  int64_t ws = fa_sm75_backward_workspace_size(&p);
   torch::Tensor work;  // released after the launch: stream-ordered reuse
   if (ws > 0) {
-    work = torch::empty({ws}, Q.options().dtype(torch::kUInt8));
+    const auto bytes = Q.options().dtype(torch::kUInt8);
+    try {
+      work = torch::empty({ws}, bytes);
+    } catch (const c10::OutOfMemoryError&) {  // the required part alone: no dK/dV split
+      ws = p.batch * p.heads_q * ((p.seq_len + 63) / 64) * 520;
+      work = torch::empty({ws}, bytes);
+    }
     p.workspace = work.data_ptr();
     p.workspace_bytes = ws;
   }

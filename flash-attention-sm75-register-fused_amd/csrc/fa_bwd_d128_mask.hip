@@ -2,6 +2,6 @@
 #include "fa_bwd_kernel.h"
 
 namespace fa {
-template void launch_bwd<128, false, true>(const BwdArgs&, int, bool, hipStream_t);
-template void launch_bwd<128, true, true>(const BwdArgs&, int, bool, hipStream_t);
+template void launch_bwd<128, false, true>(const BwdArgs&, const BwdSplit&, int, bool, hipStream_t);
+template void launch_bwd<128, true, true>(const BwdArgs&, const BwdSplit&, int, bool, hipStream_t);
 }  // namespace fa

@@ -115,6 +115,14 @@ __device__ __forceinline__ void direct_load4(__amdgpu_buffer_rsrc_t r, lds_void*
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 4, voff, 0, 0, 0);
 }
 
+struct BwdNoSplit {};
+// Partials of piece slot `slot` of a split: dV (role 0) or dK (role 1) of key
+// group kq, 32 keys x D dims in the accumulators' lane order.
+template <int D>
+__device__ __forceinline__ float* dkdv_part(const BwdSplit& sp, int slot, int role, int kq) {
+  return sp.part + (((int64_t)slot * 2 + role) * 4 + kq) * (32 * D);
+}
+
 // ---- dK, dV with two waves per key group -----------------------------------
 // One workgroup of 8 waves per (batch, KV head, 128 keys).  Waves w and w+4
 // (w = 0..3) own keys k0 + 32w .. +32, one key per lane, and run on the same
@@ -131,8 +139,13 @@ __device__ __forceinline__ void direct_load4(__amdgpu_buffer_rsrc_t r, lds_void*
 // step parity).  Q/dO tiles (and their stats and mask words) are triple
 // buffered: period p reads stages p and p - 1 and loads step p + 1 into the
 // third; one barrier ends each period.
-template <int D, bool CAUSAL, bool MASK, bool BF16>
-__global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
+//
+// SPLIT: a workgroup's work is a piece of its key block's steps (BwdSplit);
+// Split is BwdSplit then, and an empty struct otherwise (its tables are 1.4
+// KB of kernel arguments that launches without a split do not carry).
+template <int D, bool CAUSAL, bool MASK, bool BF16, class Split>
+__global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a, const Split sp) {
+  constexpr bool SPLIT = std::is_same<Split, BwdSplit>::value;
   using L = Lds<D>;
   using E = Elem<BF16>;
   constexpr int KK = D / 16;
@@ -167,8 +180,19 @@ __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
   const int wg = (int)blockIdx.x;
   const int x = wg % a.xcds, p = wg / a.xcds;
   const int per = a.units / a.xcds;
-  const int kb = p / per;
-  const int u = x * per + (p - kb * per);
+  const int rank = p / per;
+  const int u = x * per + (p - rank * per);
+  // SPLIT: item `rank` of the unit's list is piece `piece` of the `pieces` of
+  // key block kb, and its partials go to `slot`.
+  int kb = rank, piece = 0, pieces = 1, slot = 0;
+  if constexpr (SPLIT) {
+    const int it = sp.item[rank];
+    kb = it & 255;
+    piece = it >> 8;
+    const int first = sp.first[kb];
+    pieces = sp.first[kb + 1] - first;
+    slot = u * sp.pieces + first + piece;
+  }
   const int hkv_count = a.hq / a.group;
   const int b = u / hkv_count, hkv = u - b * hkv_count;
   const int k0 = kb * kBwdBlockKeys;
@@ -238,11 +262,21 @@ __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
       qt_hi = hi > lo ? hi : 0;
     }
   }
-  const int qt_begin =
-      max(qt_lo, CAUSAL ? min(a.qtiles, max(0, k0 - a.diag) / kBwdStatsTile) : 0);
-  const int qt_end = min(a.qtiles, qt_hi);
-  const int per_head = max(0, qt_end - qt_begin);
-  const int steps = a.group * per_head;
+  // The block's steps: query tiles a.qtiles - 1 down to qt_first, every head
+  // of the group at each; this workgroup's piece of them, and of that the
+  // steps inside the mask's query tiles.
+  const int qt_first = CAUSAL ? min(a.qtiles, max(0, k0 - a.diag) / kBwdStatsTile) : 0;
+  const int all_steps = a.group * (a.qtiles - qt_first);
+  int s_begin = 0, s_end = all_steps;
+  if (SPLIT && pieces > 1) {
+    s_begin = (int)((int64_t)piece * all_steps / pieces);
+    s_end = (int)((int64_t)(piece + 1) * all_steps / pieces);
+  }
+  if constexpr (MASK) {
+    s_begin = max(s_begin, a.group * (a.qtiles - min(a.qtiles, qt_hi)));
+    s_end = min(s_end, a.group * (a.qtiles - max(qt_first, qt_lo)));
+  }
+  const int steps = max(0, s_end - s_begin);
 
   // P-waves load the Q tile, dS-waves the dO tile (segments kq, kq+4, ..).
   int goff[SEGQ];
@@ -272,8 +306,7 @@ __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
     else if constexpr (S == 1) return m_lds1;
     else return m_lds2;
   };
-  // Steps go through the query tiles in descending order, every head of the
-  // group at each tile: a cursor (qt, h) names query tile qt of query head
+  // A cursor (qt, h) names the step of query tile qt of query head
   // hkv * group + h.
   struct Cursor {
     int qt, h;
@@ -509,8 +542,9 @@ __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
   // that publishes it (and the P of step p); the roles run separate loops
   // with the same number of barriers.
   if (steps > 0) {
-    Cursor ic{qt_end - 1, 0};  // next step to load
-    Cursor wc{qt_end - 1, 0};  // step to work on
+    const int qt_down = s_begin / a.group;
+    Cursor ic{a.qtiles - 1 - qt_down, s_begin - qt_down * a.group};  // next step to load
+    Cursor wc = ic;                                                  // step to work on
     issue(ic, I0{});
     advance(ic);
     barrier_after_loads<0>();
@@ -562,7 +596,23 @@ __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
     }
   }
 
-  if (krow < NK) {
+  bool whole = true;  // this workgroup's sums are the block's
+  if constexpr (SPLIT) whole = pieces == 1;
+  if constexpr (SPLIT) {
+    if (!whole) {
+      // fp32 partials, unscaled: per output tile, four consecutive dims of
+      // the lane's key per 16-byte slot.
+      float4v* dst = (float4v*)dkdv_part<D>(sp, slot, role, kq);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          dst[(mt * 4 + g) * 64 + lane] =
+              float4v{acc[mt][4 * g], acc[mt][4 * g + 1], acc[mt][4 * g + 2], acc[mt][4 * g + 3]};
+      }
+    }
+  }
+  if (whole && krow < NK) {
     _Float16* dst = role == 0 ? a.dv + b * a.dvsb + hkv * a.dvsh + (int64_t)krow * a.dvsn
                               : a.dk + b * a.dksb + hkv * a.dksh + (int64_t)krow * a.dksn;
     const float f = role == 0 ? 1.0f : a.scale;
@@ -576,6 +626,52 @@ __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a) {
         *(half4*)(dst + 32 * mt + 8 * g + 4 * hi) = v;
       }
     }
+  }
+}
+
+// Sums the partials of the key blocks a split gave more than one piece, in
+// piece order.  One wave per (unit, key block, dV or dK, key group, 32-dim
+// output tile); four 16-byte loads per lane and piece, the pieces' loads
+// independent of each other.
+template <int D, bool BF16>
+__global__ void __launch_bounds__(256) fa_bwd_merge_kernel(const BwdArgs a, const BwdSplit sp) {
+  using E = Elem<BF16>;
+  constexpr int MT = D / 32;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = (int)threadIdx.x & 63;
+  const int hi = lane >> 5, ql = lane & 31;
+  int w = (int)blockIdx.x * 4 + wave;  // (unit, merged block, role, key group, output tile)
+  const int mt = w % MT;
+  w /= MT;
+  const int kq = w & 3, role = (w >> 2) & 1;
+  w >>= 3;
+  const int u = w / sp.merged;
+  const int kb = sp.merge[w - u * sp.merged];
+  const int first = sp.first[kb], n = sp.first[kb + 1] - first;
+  const int64_t piece = 8 * 32 * D / 4;  // float4s from one piece to the next
+  const float4v* src =
+      (const float4v*)dkdv_part<D>(sp, u * sp.pieces + first, role, kq) + mt * 256 + lane;
+  float4v acc[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) acc[g] = src[g * 64];
+#pragma unroll 4
+  for (int i = 1; i < n; ++i) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] += src[i * piece + g * 64];
+  }
+  const int hkv_count = a.hq / a.group;
+  const int b = u / hkv_count, hkv = u - b * hkv_count;
+  const int krow = kb * kBwdBlockKeys + 32 * kq + ql;
+  if (krow >= a.nk) return;
+  _Float16* dst = role == 0 ? a.dv + b * a.dvsb + hkv * a.dvsh + (int64_t)krow * a.dvsn
+                            : a.dk + b * a.dksb + hkv * a.dksh + (int64_t)krow * a.dksn;
+  const float f = role == 0 ? 1.0f : a.scale;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    half4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = E::round(acc[g][e] * f);
+    *(half4*)(dst + 32 * mt + 8 * g + 4 * hi) = v;
   }
 }
 
@@ -817,28 +913,40 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
 
 }  // namespace
 
-// Launches the two backward kernels for head dimension D (the launcher in
+// Launches the backward kernels for head dimension D (the launcher in
 // fa_bwd.hip has planned the grids).
 template <int D, bool BF16, bool MASK>
-void launch_bwd(const BwdArgs& a, int batch, bool causal, hipStream_t stream) {
-  const int dkdv_wgs = a.units * ((a.nk + kBwdBlockKeys - 1) / kBwdBlockKeys);
+void launch_bwd(const BwdArgs& a, const BwdSplit& split, int batch, bool causal,
+                hipStream_t stream) {
+  const int key_blocks = (a.nk + kBwdBlockKeys - 1) / kBwdBlockKeys;
+  const int dkdv_wgs = a.units * (split.pieces > 0 ? split.pieces : key_blocks);
   const int dq_wgs = a.items;
   // dQ first: it writes the row statistics the dK/dV kernel reads (its grid
   // covers every query row, a.items = batch * heads * ceil(n / 128)).
-  if (causal) {
-    if (dq_wgs > 0)
-      hipLaunchKernelGGL((fa_bwd_dq_kernel<D, true, MASK, BF16>), dim3(dq_wgs), dim3(256), 0, stream,
-                         a);
-    if (dkdv_wgs > 0)
-      hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, true, MASK, BF16>), dim3(dkdv_wgs), dim3(512), 0,
+  if (dq_wgs > 0) {
+    if (causal)
+      hipLaunchKernelGGL((fa_bwd_dq_kernel<D, true, MASK, BF16>), dim3(dq_wgs), dim3(256), 0,
                          stream, a);
-  } else {
-    if (dq_wgs > 0)
-      hipLaunchKernelGGL((fa_bwd_dq_kernel<D, false, MASK, BF16>), dim3(dq_wgs), dim3(256), 0, stream,
-                         a);
-    if (dkdv_wgs > 0)
-      hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, false, MASK, BF16>), dim3(dkdv_wgs), dim3(512), 0,
+    else
+      hipLaunchKernelGGL((fa_bwd_dq_kernel<D, false, MASK, BF16>), dim3(dq_wgs), dim3(256), 0,
                          stream, a);
+  }
+  auto dkdv = [&](const auto& sp) {
+    using Split = std::decay_t<decltype(sp)>;
+    if (causal)
+      hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, true, MASK, BF16, Split>), dim3(dkdv_wgs),
+                         dim3(512), 0, stream, a, sp);
+    else
+      hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, false, MASK, BF16, Split>), dim3(dkdv_wgs),
+                         dim3(512), 0, stream, a, sp);
+  };
+  if (split.pieces > 0) dkdv(split);
+  else if (dkdv_wgs > 0) dkdv(BwdNoSplit{});
+  if (split.pieces > 0 && split.merged > 0) {
+    // Four waves per workgroup; 8 * D / 32 waves per (unit, block): a multiple of four.
+    const int waves = a.units * split.merged * 8 * (D / 32);
+    hipLaunchKernelGGL((fa_bwd_merge_kernel<D, BF16>), dim3(waves / 4), dim3(256), 0, stream, a,
+                       split);
   }
 }
 

@@ -339,6 +339,32 @@ int validate_bwd(const fa_bwd_params* p) {
   return FA_OK;
 }
 
+// Offset of the dK/dV split's partials in the backward's workspace.
+int64_t bwd_part_offset(const fa_bwd_params* p) {
+  return (fa::bwd_workspace_bytes(p->batch, p->heads_q, p->seq_len) + 255) / 256 * 256;
+}
+
+// The dK/dV split of a call and the bytes of its partials (0: no split, also
+// for parameters the call would be refused for).
+int64_t bwd_split(const fa_bwd_params* p, fa::BwdSplit& split) {
+  split.pieces = 0;
+  split.merged = 0;
+  split.part = nullptr;
+  const int64_t nk = bwd_kv_rows(p);
+  if (p->batch <= 0 || p->heads_kv <= 0 || p->heads_q <= 0 || p->heads_q % p->heads_kv != 0 ||
+      p->seq_len <= 0 || nk <= 0 || p->seq_len > INT32_MAX / 2 || nk > INT32_MAX / 2 ||
+      p->batch * p->heads_q >= (1 << 24) || (p->head_dim != 64 && p->head_dim != 128))
+    return 0;
+  fa::BwdArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.n = (int)p->seq_len;
+  a.nk = (int)nk;
+  a.diag = p->causal == FA_CAUSAL_BOTTOM_RIGHT ? a.nk - a.n : 0;
+  a.hq = (int)p->heads_q;
+  a.group = (int)(p->heads_q / p->heads_kv);
+  return fa::plan_bwd_split(a, (int)p->batch, (int)p->head_dim, p->causal != FA_CAUSAL_NONE, split);
+}
+
 }  // namespace
 
 // Scratch of fa_sm75_forward_noalloc: the split-K partials or the dynamic
@@ -583,14 +609,28 @@ int fa_sm75_backward(const fa_bwd_params* p) {
   a.group = (int)(p->heads_q / p->heads_kv);
   a.c2 = p->scale * 1.4426950408889634f;
   a.scale = p->scale;
-  fa::launch_backward(a, (int)p->batch, (int)p->head_dim, p->causal != FA_CAUSAL_NONE,
+  // The split's partials follow the required part of the workspace; without
+  // room for them (or rows to sum over) every key block is one workgroup's.
+  fa::BwdSplit split;
+  const int64_t part = bwd_split(p, split);
+  if (part > 0) {
+    const int64_t ofs = bwd_part_offset(p);
+    if (p->workspace_bytes >= ofs + part)
+      split.part = reinterpret_cast<float*>(static_cast<char*>(p->workspace) + ofs);
+    else
+      split.pieces = 0;
+  }
+  fa::launch_backward(a, split, (int)p->batch, (int)p->head_dim, p->causal != FA_CAUSAL_NONE,
                       p->dtype == FA_DTYPE_BF16, reinterpret_cast<hipStream_t>(p->stream));
   return check_launch();
 }
 
 int64_t fa_sm75_backward_workspace_size(const fa_bwd_params* p) {
   if (p == nullptr || p->batch < 0 || p->heads_q < 0 || p->seq_len < 0) return 0;
-  return fa::bwd_workspace_bytes(p->batch, p->heads_q, p->seq_len);
+  const int64_t need = fa::bwd_workspace_bytes(p->batch, p->heads_q, p->seq_len);
+  fa::BwdSplit split;
+  const int64_t part = bwd_split(p, split);
+  return part > 0 ? bwd_part_offset(p) + part : need;
 }
 
 const char* fa_sm75_last_error(void) { return g_last_error; }

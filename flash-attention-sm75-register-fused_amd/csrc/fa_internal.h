@@ -209,8 +209,32 @@ struct BwdArgs {
 constexpr int kBwdStatsTile = 64;    // query rows per stats record
 constexpr int kBwdBlockKeys = 128;   // keys per dK/dV workgroup
 constexpr int kBwdBlockRows = 128;   // query rows per dQ workgroup
-// Workspace bytes of a backward call: the statistics records, then the
-// query tiles' key spans (BwdArgs::stats, tspans).
+// Split of the dK/dV kernel's key blocks over workgroups.  A key block's work
+// is a sequence of steps (one 64-row query tile of one query head each, query
+// tiles in descending order, the group's heads at each); a block of n > 1
+// pieces gives piece i the steps [i S / n, (i + 1) S / n), each piece's dK and
+// dV go to the workspace as fp32 partials and fa_bwd_merge_kernel sums them in
+// piece order.  The step ranges come from the causal bound alone, so calls
+// with and without mask ranges sum in the same grouping.  Every unit (batch,
+// KV head) has the same list, which the launcher passes with the kernel
+// arguments.
+constexpr int kBwdMaxPieces = 512;     // per unit
+constexpr int kBwdMaxSplitBlocks = 128;  // key blocks per unit
+struct BwdSplit {
+  int pieces;     // work items per unit, largest first (0: one per key block, no split)
+  int merged;     // key blocks with more than one piece
+  float* part;    // [units * pieces][2][128 * D] fp32 partials (see dkdv_part)
+  uint16_t item[kBwdMaxPieces];           // key block | piece << 8
+  uint16_t first[kBwdMaxSplitBlocks + 1]; // first piece slot of each key block
+  uint8_t merge[kBwdMaxSplitBlocks];      // the key blocks with more than one piece
+};
+// Plans the split of a call (a: n, nk, diag, hq, group set); s.pieces is 0
+// where one workgroup per key block is faster.  Returns the bytes of s.part.
+int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, BwdSplit& s);
+
+// Workspace bytes a backward call requires: the statistics records, then the
+// query tiles' key spans (BwdArgs::stats, tspans).  The split's partials
+// follow at the next multiple of 256 bytes when the workspace has room.
 inline int64_t bwd_stats_bytes(int64_t batch, int64_t heads_q, int64_t seq_len) {
   return batch * heads_q * ((seq_len + kBwdStatsTile - 1) / kBwdStatsTile) *
          (2 * kBwdStatsTile) * (int64_t)sizeof(float);
@@ -220,11 +244,13 @@ inline int64_t bwd_workspace_bytes(int64_t batch, int64_t heads_q, int64_t seq_l
          batch * heads_q * ((seq_len + kBwdStatsTile - 1) / kBwdStatsTile) * 2 *
              (int64_t)sizeof(int32_t);
 }
-// Launches the dQ and dK/dV kernels; all arguments validated.
-int launch_backward(const BwdArgs& a, int batch, int head_dim, bool causal, bool bf16,
-                    hipStream_t stream);
+// Launches the dQ and dK/dV kernels (and, for a split, the merge); all
+// arguments validated.
+int launch_backward(const BwdArgs& a, const BwdSplit& split, int batch, int head_dim, bool causal,
+                    bool bf16, hipStream_t stream);
 template <int D, bool BF16, bool MASK>
-void launch_bwd(const BwdArgs& a, int batch, bool causal, hipStream_t stream);
+void launch_bwd(const BwdArgs& a, const BwdSplit& split, int batch, bool causal,
+                hipStream_t stream);
 
 // Boolean mask -> bit rows (fa_mask.hip); ranges (or nullptr): each row's
 // first visible key and one past the last ([cols, 0] for none), int32 pairs.

@@ -287,9 +287,10 @@ typedef struct fa_bwd_params {
   int causal;           /* an fa_causal value (the forward's) */
   int dtype;            /* an fa_dtype */
   void* stream;         /* hipStream_t; NULL selects the default stream */
-  void* workspace;      /* device scratch of at least
-                           fa_sm75_backward_workspace_size() bytes, 16-byte
-                           aligned (required); calls that share one race */
+  void* workspace;      /* device scratch, 16-byte aligned: 520 bytes per
+                           (batch, query head, 64 query rows) are required,
+                           fa_sm75_backward_workspace_size() are used; calls
+                           that share one race */
   int64_t workspace_bytes;
   /* Optional explicit mask, or NULL: the forward's (fa_fwd_params.mask_bits,
    * same bit layout and word strides, 0 broadcasts a dimension); combines
@@ -308,14 +309,19 @@ typedef struct fa_bwd_params {
 void fa_sm75_set_contiguous_bwd_strides(fa_bwd_params* p);
 
 /* Backward: two kernels on p->stream (dQ, which also writes per-row
- * statistics into the workspace, then dK/dV).  Asynchronous; validates every argument
- * before touching the device.  Returns FA_OK or an fa_status. */
+ * statistics into the workspace, then dK/dV), and a third that sums dK/dV
+ * partials where the workspace holds them.  Asynchronous; validates every
+ * argument before touching the device.  Returns FA_OK or an fa_status. */
 int fa_sm75_backward(const fa_bwd_params* p);
 
-/* Workspace bytes fa_sm75_backward needs: 520 per (batch, query head, 64
+/* Workspace bytes fa_sm75_backward uses: 520 per (batch, query head, 64
  * query rows) -- that tile's row statistics, then its span of visible keys
- * when mask_ranges is given -- from batch, heads_q and seq_len alone (0 if
- * one is negative or p is NULL). */
+ * when mask_ranges is given -- which are required, and, where one dK/dV
+ * workgroup per 128 keys would leave CUs idle, room (at most 134 MB) for the
+ * fp32 partials of several per 128 keys.  With less than that the call runs
+ * with one.  From the sizes, head_dim and causal flag alone (0 if a size is
+ * negative or p is NULL; the required bytes if they are not a valid call's).
+ * The same call with the same workspace size gives the same bits. */
 int64_t fa_sm75_backward_workspace_size(const fa_bwd_params* p);
 
 #define FA_SM75_ABI_VERSION 7
