@@ -16,8 +16,9 @@
 //   * the four waves' (max, sum, O) merge through LDS at the end;
 //   * with one split the workgroup writes O (and LSE) directly; otherwise it
 //     writes an fp32 partial (unnormalised O, running max in log2 units, sum)
-//     to the caller's workspace and fa_decode_combine (for many splits,
-//     fa_decode_combine_wide) merges the splits.
+//     to the caller's workspace, and the unit's last workgroup to finish
+//     merges them (MERGE) or, where they are many bytes, fa_decode_combine
+//     (for many splits, fa_decode_combine_wide) does in a second launch.
 //
 // Small launches (a 128-row prefill grid of at most kSmallLaunchItems
 // workgroups, e.g. one head of 512 rows) take the same path with the query
@@ -35,6 +36,8 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 
 #include "fa_internal.h"
 
@@ -44,15 +47,6 @@ namespace fa {
 namespace {
 
 constexpr int kDecTile = 32;       // keys per wave tile
-constexpr int kDecMinTiles = 8;    // fewest tiles a split is given (decode)
-constexpr int kSmallMinTiles = 4;  // small launches: one tile per wave
-// Small launches with at most this many 32-key tiles run one split per unit:
-// the four waves of the workgroup (16 tiles each at most) are then the whole
-// key split, and the launch needs neither a workspace nor the combine kernel
-// (whose launch costs more than it saves on such short key ranges; measured
-// on MI355X: one head of 512 rows 6.3 against 8.9 us, of 2048 rows even).
-constexpr int kSmallNoSplitTiles = 64;
-constexpr int kDecTargetWgs = 256; // one workgroup per CU (measured best)
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
@@ -91,11 +85,57 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("" ::: "memory");
 }
 
+// Cache policy of the in-kernel merge's accesses: sc1, coherent over the
+// device's L2s.
+constexpr int kCoherent = 16;
+// 16-byte partials a merging thread has in flight at once.
+constexpr int kMergeLoads = 8;
+// Units with at most this many bytes of partial O are merged by the split-K
+// kernel itself: it saves the second launch (3.1 us of host time, and 0-0.5
+// us on the GPU: Hq=14 Hkv=2 d64 4097 keys 9.0 -> 8.6 us back to back, 11.0 ->
+// 8.7 through the SDPA patch, where the host is the limit).  One workgroup
+// reads a unit's partials at about 50 bytes/ns, so larger ones go to the
+// combine kernels' many (Hq=32 Hkv=8 8 rows 2048 keys d128, 128 KB: 14.8 us
+// merged here, 11.1 by the combine kernel; 64 KB within 0.7 us either way).
+constexpr int kMergeMaxBytes = 64 << 10;
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Normalises and stores 4 dimensions of query column c of row block rb of
+// (batch, KV head) bh from the splits' merged max (log2 units), sum and O,
+// and the row's LSE once.  Columns past the last row are not stored.
+template <int D, bool BF16>
+__device__ __forceinline__ void store_merged(const DecArgs& d, int bh, int rb, int c, int dim,
+                                             float m, float l, v4f o) {
+  const FwdArgs& a = d.f;
+  const int hkv_count = a.hq / a.group;
+  const int b = bh / hkv_count;
+  const int hkv = bh - b * hkv_count;
+  const int r = rb * kDecodeMaxRows + c;
+  if (r >= d.total_rows) return;
+  const int g = r / a.n;
+  const int qi = r - g * a.n;
+  const int hq = hkv * a.group + g;
+  const float inv = (l > 0.0f) ? (1.0f / l) : 0.0f;
+  half4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = Elem<BF16>::round(o[e] * inv);
+  *(half4*)(a.o + b * a.osb + hq * a.osh + (int64_t)qi * a.osn + dim) = v;
+  if (a.lse != nullptr && dim == 0) {
+    const float m_use = (m == -__builtin_inff()) ? 0.0f : m;
+    a.lse[((int64_t)b * a.hq + hq) * a.n + qi] =
+        (m_use + __builtin_log2f(l)) * 0.69314718055994530942f;
+  }
+}
+
 // MASK_MODE: 0 no explicit mask, 1 mask bits (one 32-bit word per row and
 // tile), 2 key-padding bytes (fa_fwd_params.mask_keys: one byte per key, the
 // same for every row of the batch; a ballot over the tile's 32 bytes forms
-// the word).
-template <int D, bool CAUSAL, int MASK_MODE, bool BF16>
+// the word).  MERGE: the unit's last workgroup merges its splits (an instance
+// of its own: with that code in it the others' tile loop ran up to 13%
+// slower, one head of 256 rows of 8 at head_dim 64 5.0 -> 5.6 us).
+template <int D, bool CAUSAL, int MASK_MODE, bool BF16, bool MERGE>
 __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d) {
   constexpr bool MASK = MASK_MODE != 0;
   constexpr bool KEY_BYTES = MASK_MODE == 2;
@@ -409,8 +449,10 @@ __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d)
     ml[64 + lane] = l_tot;
   }
   __syncthreads();
-  if (wave >= MT) return;
-  const int mt = wave;  // this wave merges output tile mt
+  // Wave mt merges output tile mt (at head_dim 64 waves 2 and 3 have none, and
+  // go on only for the splits' merge).
+  if (!MERGE && wave >= MT) return;
+  const int mt = wave < MT ? wave : 0;
   float m_w[kWaves], M = -__builtin_inff();
 #pragma unroll
   for (int u = 0; u < kWaves; ++u) {
@@ -432,8 +474,9 @@ __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[i] += f * base[i * 64 + lane];
   }
-  if (!row_ok) return;
-  if (d.splits == 1) {
+  const bool mine = row_ok && wave < MT;
+  if (!MERGE && !mine) return;
+  if (!MERGE && d.splits == 1) {
     const float inv = (Ltot > 0.0f) ? (1.0f / Ltot) : 0.0f;
     _Float16* op = a.o + b * a.osb + hq * a.osh + (int64_t)qi * a.osn + 32 * mt + 4 * hi;
 #pragma unroll
@@ -448,7 +491,10 @@ __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d)
       a.lse[((int64_t)b * a.hq + hq) * nq + qi] =
           (m_use * c2 + __builtin_log2f(Ltot)) * 0.69314718055994530942f;
     }
-  } else {
+    return;
+  }
+  const float M2 = (M == -__builtin_inff()) ? M : M * c2;  // log2 units
+  if constexpr (!MERGE) {  // a combine kernel merges the splits
     const int64_t p = ((int64_t)unit * d.splits + split) * d.rows + ql;
     float* po = d.part_o + p * D + 32 * mt + 4 * hi;
 #pragma unroll
@@ -457,9 +503,145 @@ __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d)
       *(float4*)(po + 8 * g4) = v;
     }
     if (mt == 0 && hi == 0) {
-      d.part_ml[2 * p] = (M == -__builtin_inff()) ? -__builtin_inff() : M * c2;
+      d.part_ml[2 * p] = M2;
       d.part_ml[2 * p + 1] = Ltot;
     }
+    return;
+  }
+
+  if constexpr (MERGE) {
+    // ---- merge of the unit's splits by the last workgroup to finish ----------
+    // Every partial and flag goes through device-coherent accesses (the sc1
+    // bit: stores write through to memory, loads do not take a line another
+    // XCD's L2 may have left stale), so no cache has to be written back or
+    // invalidated: a release fence here would write back the XCD's whole L2
+    // (20-35% of a call, measured).  A workgroup's partials are acknowledged
+    // before it sets its flag, and its flag before it reads the others', so of
+    // any two workgroups of a unit at least one sees the other's flag set, and
+    // the last flag to be set is set by a workgroup that sees them all.  Two that
+    // both see all of them merge the same partials in the same order and store
+    // the same values.
+    const int unit_ml = unit * d.splits * d.rows;  // first (split, row) record of the unit
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc(d.part_o + (int64_t)unit_ml * D, d.splits * d.rows * D * 4);
+    const __amdgpu_buffer_rsrc_t rl = make_rsrc(d.part_ml + (int64_t)unit_ml * 2, d.splits * d.rows * 8);
+    const __amdgpu_buffer_rsrc_t rf = make_rsrc(d.flags + (int64_t)unit * d.splits, d.splits * 8);
+    if (mine) {
+      const int rec = split * d.rows + ql;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const v4f v = {o[4 * g4], o[4 * g4 + 1], o[4 * g4 + 2], o[4 * g4 + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), rp,
+                                               (rec * D + 32 * mt + 4 * hi + 8 * g4) * 4, 0, kCoherent);
+      }
+      if (mt == 0 && hi == 0)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v2f{M2, Ltot}), rl, rec * 8, 0,
+                                              kCoherent);
+    }
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (tid == 0) {
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, d.mark), rf, split * 8, 0, kCoherent);
+      wait_vmcnt<0>();
+    }
+    __syncthreads();
+    bool set = true;  // one flag per thread (at most kThreads splits)
+    if (tid < d.splits)
+      set = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(rf, tid * 8, 0, kCoherent)) ==
+            d.mark;
+    if (!__syncthreads_and(set)) return;
+
+    // Thread (grp, item): 4 dimensions of one query column (item = column *
+    // D / 4 + dimension / 4), splits grp, grp + groups, ...; the groups' states
+    // meet in LDS.  More than kThreads items: one group, items in turns.
+    const int items = d.rows * (D / 4);
+    const int groups = max(1, min(kThreads / items, d.splits));
+    const int grp_m = groups > 1 ? tid / items : 0;
+    float* const xm = ml_lds;              // [group][item] max, then sum (kThreads each)
+    float4* const xo = (float4*)v_lds0;    // [group][item] O
+    static_assert(kThreads * 16 <= kWaves * L::Tile * 2, "the merge's states fit the V tiles");
+    // NI items at once (kThreads apart), so that a thread with several has all
+    // their loads in flight together.
+    auto merge = [&](int it0, auto ni_c) {
+      constexpr int NI = decltype(ni_c)::value;
+      constexpr int BATCH = kMergeLoads / NI;
+      float m_acc[NI], l_acc[NI];
+      v4f o_acc[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        m_acc[i] = -__builtin_inff();
+        l_acc[i] = 0.0f;
+        o_acc[i] = (v4f)0.0f;
+      }
+      for (int s0 = grp_m; s0 < d.splits; s0 += BATCH * groups) {
+        v4f os[NI][BATCH];
+        v2f ml[NI][BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            // Splits past the last read zeros beyond the windows (their max is
+            // replaced below).
+            const int it = it0 + i * kThreads;
+            const int rec = (s0 + u * groups) * d.rows + it / (D / 4);
+            ml[i][u] =
+                __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(rl, rec * 8, 0, kCoherent));
+            os[i][u] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   rp, (rec * D + 4 * (it % (D / 4))) * 4, 0, kCoherent));
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          float m_new = m_acc[i];
+#pragma unroll
+          for (int u = 0; u < BATCH; ++u) {
+            if (s0 + u * groups >= d.splits) ml[i][u][0] = -__builtin_inff();
+            m_new = fmaxf(m_new, ml[i][u][0]);
+          }
+          if (m_new == -__builtin_inff()) continue;
+          const float alpha = __builtin_amdgcn_exp2f(m_acc[i] - m_new);
+          l_acc[i] *= alpha;
+          o_acc[i] *= alpha;
+#pragma unroll
+          for (int u = 0; u < BATCH; ++u) {
+            const float w = __builtin_amdgcn_exp2f(ml[i][u][0] - m_new);
+            l_acc[i] += w * ml[i][u][1];
+            o_acc[i] += w * os[i][u];
+          }
+          m_acc[i] = m_new;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int it = it0 + i * kThreads;
+        if (groups > 1) {
+          xm[tid] = m_acc[i];
+          xm[kThreads + tid] = l_acc[i];
+          xo[tid] = __builtin_bit_cast(float4, o_acc[i]);
+        } else {
+          store_merged<D, BF16>(d, bh, rb, it / (D / 4), 4 * (it % (D / 4)), m_acc[i], l_acc[i], o_acc[i]);
+        }
+      }
+    };
+    int it = tid - grp_m * items;
+    if (grp_m < groups) {
+      for (; it + kThreads < items; it += 2 * kThreads) merge(it, std::integral_constant<int, 2>{});
+      if (it < items) merge(it, std::integral_constant<int, 1>{});
+    }
+    if (groups == 1) return;
+    __syncthreads();
+    if (tid >= items) return;
+    float Mg = xm[tid];
+    for (int q = 1; q < groups; ++q) Mg = fmaxf(Mg, xm[q * items + tid]);
+    float lg = 0.0f;
+    v4f og = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (Mg != -__builtin_inff()) {
+      for (int q = 0; q < groups; ++q) {
+        const float w = __builtin_amdgcn_exp2f(xm[q * items + tid] - Mg);
+        lg += w * xm[kThreads + q * items + tid];
+        og += w * __builtin_bit_cast(v4f, xo[q * items + tid]);
+      }
+    }
+    store_merged<D, BF16>(d, bh, rb, tid / (D / 4), 4 * (tid % (D / 4)), Mg, lg, og);
   }
 }
 
@@ -690,11 +872,14 @@ void launch_decode_typed(const DecArgs& d, const DecodePlan& pl, int head_dim, b
                          hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)pl.units * pl.splits));
 #define FA_DEC(DD, C, M) \
-  hipLaunchKernelGGL((fa_decode_kernel<DD, C, M, BF16>), grid, dim3(kThreads), 0, stream, d)
+  if (d.flags != nullptr)                                                                         \
+    hipLaunchKernelGGL((fa_decode_kernel<DD, C, M, BF16, true>), grid, dim3(kThreads), 0, stream, d); \
+  else                                                                                            \
+    hipLaunchKernelGGL((fa_decode_kernel<DD, C, M, BF16, false>), grid, dim3(kThreads), 0, stream, d)
 #define FA_DEC_M(DD, C)                            \
-  if (d.f.mkeys != nullptr) FA_DEC(DD, C, 2);      \
-  else if (d.f.mbits != nullptr) FA_DEC(DD, C, 1); \
-  else FA_DEC(DD, C, 0)
+  if (d.f.mkeys != nullptr) { FA_DEC(DD, C, 2); }      \
+  else if (d.f.mbits != nullptr) { FA_DEC(DD, C, 1); } \
+  else { FA_DEC(DD, C, 0); }
   if (head_dim == 128) {
     if (causal) { FA_DEC_M(128, true); } else { FA_DEC_M(128, false); }
   } else {
@@ -702,7 +887,7 @@ void launch_decode_typed(const DecArgs& d, const DecodePlan& pl, int head_dim, b
   }
 #undef FA_DEC_M
 #undef FA_DEC
-  if (pl.splits > 1) {
+  if (pl.splits > 1 && d.flags == nullptr) {
     const bool wide = pl.splits * head_dim >= kWideCombineMin;
     const dim3 cgrid((unsigned)((int64_t)pl.units * pl.rows * (wide ? head_dim / 32 : 1)));
 #define FA_CMB(DD)                                                                          \
@@ -716,6 +901,31 @@ void launch_decode_typed(const DecArgs& d, const DecodePlan& pl, int head_dim, b
   }
 
 }
+
+}  // namespace
+
+namespace {
+
+__global__ void fa_clear_flags(uint64_t* flags, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) flags[i] = 0;
+}
+
+// A mark no other call of this process has used: a counter from a random
+// start, so that what else the workspace may hold does not equal it either.
+uint64_t fresh_mark() {
+  static std::atomic<uint64_t> next{[] {
+    // splitmix64 of the clock and this object's address
+    uint64_t x = (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() +
+                 0x9e3779b97f4a7c15ull * (uint64_t)(uintptr_t)&fa_clear_flags;
+    x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+    x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+    return (x ^ (x >> 31)) | 1u;
+  }()};
+  return next.fetch_add(2, std::memory_order_relaxed);
+}
+constexpr uint64_t kCapturedMark = 2;  // calls under capture (fresh marks are odd)
+
 
 }  // namespace
 
@@ -738,6 +948,59 @@ bool decode_eligible(const FwdArgs& a, int batch) {
   return true;
 }
 
+namespace {
+
+// How many workgroups share a unit's keys.  A workgroup (four waves) streams
+// K and V at about 50 bytes/ns however many loads it has in flight (16 KB per
+// 32-key tile at head_dim 128), so few workgroups are slow and the split
+// spreads a unit over CUs; the merge costs 2-3 us.  Timed on MI355X through
+// the C ABI, bfloat16, us per call:
+//  * few tiles run as one split: decode Hq=14 Hkv=2 d64 512 keys 5.9 against
+//    7.7 for 4 splits, Hq=32 Hkv=8 d128 256 keys 7.1 against 8.7; one head of
+//    1024 rows d64 8.2 against 8.8, two of 777 d128 13.4 against 14.4; and so
+//    do row blocks (32 columns, a longer merge) that could only be halved and
+//    have at most 64 tiles at head_dim 64 (4 heads of 1024 rows 9.6 against
+//    10.3);
+//  * a split has at least kDecMinTiles tiles, one per wave, and at head_dim
+//    64 eight where the range is long (4097 keys 8.7 against 9.0 for 32
+//    splits); row blocks eight (one head of 1024 rows d128 16.1 -> 12.9, 4
+//    heads 300 x 2000 29.6 -> 16.2);
+//  * the workgroups fill whole rounds of CUs: rounding the split count up
+//    put two workgroups on some CUs and one on others, and the launch took
+//    as long as two (B=3 Hq=32 Hkv=8 9000 keys d128: 264 workgroups 31.7,
+//    240 22.6; B=12 8192 keys 288 workgroups 92.5, 192 70.2).  Where one round
+//    leaves more than a seventh of the CUs idle, two rounds' worth (two
+//    workgroups of a CU run together) if that fills them better: the latter
+//    480 workgroups 67.4, B=20 Hq=8 3000 keys d128 160 workgroups 48.2, 480
+//    44.3.
+constexpr int kDecMinTiles = 4;
+constexpr int kDecLongTiles = 64, kDecLongMinTiles = 8;
+constexpr int kSmallMinTiles = 8;
+constexpr int kTargetWgs = 256;  // one workgroup per CU
+
+int plan_splits(const DecodePlan& pl, int head_dim) {
+  const bool blocks = pl.row_blocks > 1;
+  const int no_split = blocks ? (head_dim == 64 ? 36 : 27) : head_dim == 64 ? 20 : 12;
+  if (pl.tiles <= no_split) return 1;
+  const int min_tiles = blocks ? kSmallMinTiles
+                        : head_dim == 64 && pl.tiles > kDecLongTiles ? kDecLongMinTiles
+                                                                     : kDecMinTiles;
+  int splits = std::max(1, kTargetWgs / pl.units);
+  if (blocks) {
+    if (pl.tiles > kDecLongTiles)  // one block per CU, a long range each: halve it
+      splits = std::max(splits, std::min(2, (kTargetWgs + pl.units - 1) / pl.units));
+    else if (head_dim == 64 && splits < 4)
+      splits = 1;
+  } else {
+    const int two = 2 * kTargetWgs / pl.units;
+    if (7 * splits * pl.units < 6 * kTargetWgs && two * pl.units > 9 * splits * pl.units / 4)
+      splits = two;
+  }
+  return std::max(1, std::min(std::min(splits, kMaxSplits), pl.tiles / min_tiles));
+}
+
+}  // namespace
+
 DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
                        int64_t workspace_bytes) {
   DecodePlan pl;
@@ -749,18 +1012,19 @@ DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
   int64_t nk_eff = a.nk;
   if (causal) nk_eff = std::min<int64_t>(a.nk, std::max<int64_t>(0, (int64_t)a.n + a.diag));
   pl.tiles = (int)((nk_eff + kDecTile - 1) / kDecTile);
-  int splits = std::min((kDecTargetWgs + pl.units - 1) / pl.units, kMaxSplits);
-  splits = std::min(
-      splits, std::max(1, pl.tiles / (pl.row_blocks > 1 ? kSmallMinTiles : kDecMinTiles)));
-  splits = std::max(splits, 1);
-  if (pl.row_blocks > 1 && pl.tiles <= kSmallNoSplitTiles) splits = 1;
+  const int splits = plan_splits(pl, head_dim);
   pl.chunk_tiles = std::max(1, (pl.tiles + splits - 1) / splits);
   pl.splits = std::max(1, (pl.tiles + pl.chunk_tiles - 1) / pl.chunk_tiles);
+  pl.merge_in_kernel = pl.splits > 1 && pl.splits <= kThreads &&
+                       (int64_t)pl.splits * pl.rows * head_dim * 4 <= kMergeMaxBytes;
   pl.workspace_bytes =
-      pl.splits > 1 ? (int64_t)pl.units * pl.splits * pl.rows * (head_dim + 2) * 4 : 0;
+      pl.splits > 1 ? (int64_t)pl.units * pl.splits *
+                          (pl.rows * (head_dim + 2) * 4 + (pl.merge_in_kernel ? 8 : 0))
+                    : 0;
   if (pl.workspace_bytes > workspace_bytes) {  // not enough room: one split
     pl.splits = 1;
     pl.chunk_tiles = std::max(1, pl.tiles);
+    pl.merge_in_kernel = false;
     pl.workspace_bytes = 0;
   }
   return pl;
@@ -780,6 +1044,21 @@ int launch_decode_forward(const FwdArgs& a, const DecodePlan& pl, int head_dim, 
   d.part_ml = pl.splits > 1
                   ? d.part_o + (int64_t)pl.units * pl.splits * pl.rows * head_dim
                   : nullptr;
+  d.flags = nullptr;
+  d.mark = kCapturedMark;
+  if (pl.merge_in_kernel) {
+    d.flags = reinterpret_cast<uint64_t*>(d.part_ml + (int64_t)pl.units * pl.splits * pl.rows * 2);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(stream, &capture);
+    if (e != hipSuccess) (void)hipGetLastError();  // not this call's error
+    if (e == hipSuccess && capture == hipStreamCaptureStatusNone) {
+      d.mark = fresh_mark();
+    } else {
+      const int64_t n = (int64_t)pl.units * pl.splits;
+      hipLaunchKernelGGL(fa_clear_flags, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
+                         d.flags, n);
+    }
+  }
   if (a.bf16)
     launch_decode_typed<true>(d, pl, head_dim, causal, stream);
   else

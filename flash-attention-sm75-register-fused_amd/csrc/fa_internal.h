@@ -144,9 +144,17 @@ struct DecArgs {
   int tiles;        // 32-key tiles any row can see
   float* part_o;    // [units, splits, rows, D] unnormalised O (splits > 1)
   float* part_ml;   // [units, splits, rows, 2]: max (log2 units), sum
+  // In-kernel merge (merge_in_kernel), else nullptr: one word per (unit,
+  // split), which that split's workgroup sets to `mark` once its partials are
+  // written.  No other call's mark equals this one's, so the words need no
+  // clearing (a call under stream capture clears them: its graph may run
+  // again with the same mark).
+  uint64_t* flags;
+  uint64_t mark;
 };
 struct DecodePlan {
   int rows, total_rows, row_blocks, units, tiles, splits, chunk_tiles;
+  bool merge_in_kernel;     // the split-K kernel merges the splits itself
   int64_t workspace_bytes;  // 0 when splits == 1
 };
 bool decode_eligible(const FwdArgs& a, int batch);

@@ -154,8 +154,8 @@ int64_t fa_sm75_workspace_size(const fa_fwd_params* p);
 
 /* Bytes of device scratch fa_sm75_forward_noalloc holds per GPU: the largest
  * workspace fa_sm75_workspace_size() can ask for (split-K partials of at most
- * 510 workgroups x 32 query rows x (128 + 2) floats, 8486400 bytes), rounded
- * up to 8.5 MiB. */
+ * 512 workgroups x (32 query rows x (128 + 2) floats + an 8-byte mark),
+ * 8523776 bytes), rounded up to 8.5 MiB. */
 #define FA_SM75_NOALLOC_SCRATCH_BYTES (17u << 19)
 
 /* fa_sm75_forward without a caller workspace and without any allocation: the
