@@ -40,6 +40,7 @@
 #include <chrono>
 
 #include "fa_internal.h"
+#include "flash_attn_sm75.h"
 
 #include "fa_kernel_common.h"
 
@@ -1017,10 +1018,17 @@ DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
   pl.splits = std::max(1, (pl.tiles + pl.chunk_tiles - 1) / pl.chunk_tiles);
   pl.merge_in_kernel = pl.splits > 1 && pl.splits <= kThreads &&
                        (int64_t)pl.splits * pl.rows * head_dim * 4 <= kMergeMaxBytes;
-  pl.workspace_bytes =
-      pl.splits > 1 ? (int64_t)pl.units * pl.splits *
-                          (pl.rows * (head_dim + 2) * 4 + (pl.merge_in_kernel ? 8 : 0))
-                    : 0;
+  pl.workspace_bytes = 0;
+  if (pl.splits > 1) {
+    // Partials, then the marks in whole records of one split (a size of that
+    // many splits more), or alone where those would not fit the no-allocation
+    // entry's scratch.
+    const int64_t record = (int64_t)pl.units * pl.rows * (head_dim + 2) * 4;
+    const int64_t marks = pl.merge_in_kernel ? (int64_t)pl.units * pl.splits * 8 : 0;
+    pl.workspace_bytes = record * (pl.splits + (marks + record - 1) / record);
+    if (pl.workspace_bytes > (int64_t)FA_SM75_NOALLOC_SCRATCH_BYTES)
+      pl.workspace_bytes = record * pl.splits + marks;
+  }
   if (pl.workspace_bytes > workspace_bytes) {  // not enough room: one split
     pl.splits = 1;
     pl.chunk_tiles = std::max(1, pl.tiles);
