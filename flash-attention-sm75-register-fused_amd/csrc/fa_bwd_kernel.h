@@ -108,8 +108,6 @@ __device__ __forceinline__ void put_pair(uint4v (&ops)[NOPS], int t, int i, floa
   ops[2 * t + (i >> 3)][(i & 7) >> 1] = __builtin_bit_cast(unsigned, E::pack(x, y));
 }
 
-typedef float float4v __attribute__((ext_vector_type(4)));
-
 // 4-byte direct load of one lane (lane l writes dst + 4 l).
 __device__ __forceinline__ void direct_load4(__amdgpu_buffer_rsrc_t r, lds_void* dst, int voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 4, voff, 0, 0, 0);

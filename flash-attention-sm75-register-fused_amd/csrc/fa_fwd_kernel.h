@@ -88,19 +88,22 @@ namespace {
 // 64-bit word per query row and tile, loaded a step ahead) hides keys too;
 // MASK_MODE 2: a key-padding mask read as bytes (one per lane and tile, loaded
 // a step ahead; a ballot over the wave forms the same word).
-// ROWSUM: the row sums of P come from the matrix pipe, as one more 32-row
-// output tile of O^T whose A operand is a row of ones (4 more MFMAs and 16
-// fewer VALU instructions per tile).  Launched for head_dim-64 causal
-// launches that hold every block at once: there a CU's large block runs its
-// last tiles alone, one wave per SIMD, and its step latency is the launch's
-// tail (measured: C3 +3.4%, B=1 Hq=14 Hkv=2 N=4096 +4.8%; launches that keep
-// two waves per SIMD busy throughout lose 1-2%, the extra matrix work costing
-// clock).
+// ROWSUM (head_dim 64): the row sums of P come from the matrix pipe, four
+// 16x16x32 MFMAs per tile whose A operand is ones (each sums 16 keys of all 32
+// queries) in place of 16 v_dot2: a head_dim-64 step is bound by its VALU
+// work, and these MFMAs take a quarter of a 32x32x16 tile's four each.  Every
+// head_dim-64 launch has it except non-causal ones of several rounds without
+// a mask, whose matrix pipe has no time left (interleaved A/B on
+// MI355X, with against without, us: B=4 H=12 N=1024 full 20.8 / 21.2, B=3
+// Hq=14 Hkv=2 N=1777 causal 27.3 / 28.2, B=1 Hq=32 Hkv=8 N=8192 causal 303 /
+// 312, B=2 Hq=64 Hkv=8 N=16384 causal 4593 / 4756, B=2 H=8 N=4096 full, one
+// round, 75.2 / 77.2; but B=2 H=24 N=1500 full 44.2 / 42.2, B=8 H=16 N=1024
+// full 44.9 / 43.5).
 // DYN: the instance carries the dynamic schedule's item loop (4-wave launches
 // that run it).  Static launches take instances without it: the loop's
 // claim, prefetch and hand-off state costs registers all through the steps
-// (the ROWSUM instance: 106 SGPRs spilled to VGPR lanes and 232 VGPRs with
-// it, 15 and 222 without; C3 1.033-1.040x, results bitwise unchanged).
+// (a causal head_dim-64 instance: 106 SGPRs spilled to VGPR lanes and 232
+// VGPRs with it, 15 and 222 without; C3 1.033-1.040x, results bitwise unchanged).
 // LDS through which group 1 of a key split hands its share of a block to
 // group 0: per row wave, MT * 1024 floats of O (four consecutive floats of a
 // lane's accumulator per 16-byte slot), then 64 running maxima and 64 lane
@@ -120,7 +123,8 @@ __device__ __forceinline__ float* pair_exchange() {
 template <int D, bool CAUSAL, bool KV_SAME_STRIDE, int WAVES, int MASK_MODE, bool KSPLIT, bool BF16,
           bool ROWSUM, bool DYN>
 __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) {
-  static_assert(!DYN || (WAVES == 4 && !ROWSUM), "the dynamic schedule runs on 4-wave instances");
+  static_assert(!DYN || WAVES == 4, "the dynamic schedule runs on 4-wave instances");
+  static_assert(!ROWSUM || D == 64, "row sums from the matrix pipe: head_dim 64");
   constexpr bool MASK = MASK_MODE != 0;        // an explicit mask: bits or key bytes
   constexpr bool KEY_BYTES = MASK_MODE == 2;   // key-padding bytes (a.mkeys)
   // LDS tile layout: dense (no row padding, 8 direct loads per tile instead
@@ -132,9 +136,9 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
   using E = Elem<BF16>;
   constexpr int KK = D / 16;       // 16-wide contraction steps of S^T
   constexpr int MT = D / 32;       // 32-row output tiles of O^T
-  constexpr int MTX = MT + (ROWSUM ? 1 : 0);  // P V output tiles, the row-sum tile last
   constexpr int NS = 2 * KK;       // S^T MFMAs per tile
-  constexpr int NPV = 4 * MTX;     // P V MFMAs per tile
+  constexpr int MTX = MT + (ROWSUM ? 1 : 0);  // MFMA slots of a 16-key P V step, the row sums' last
+  constexpr int NPV = 4 * MTX;     // P V slots per tile
   constexpr int PFK = 3;           // K operand reads run this many MFMAs ahead
   constexpr int PFV = 2;           // V operand reads run this many MFMAs ahead
   constexpr int ROW_WAVES = KSPLIT ? 4 : WAVES;  // waves owning distinct rows
@@ -521,14 +525,16 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
       const int off = ((kk & 1) ? k_base_odd : k_base_even) + 32 * t * L::Pitch + 32 * (kk >> 1);
       return *(const half8*)(Ks + off);
     };
-    // A operand of the row-sum tile (ROWSUM): row 0 all ones (lanes 0 and 32
-    // hold its two 8-key halves), rows 1-31 zero.  Row 0 of that tile's
-    // accumulator, lane c's register 0, is query c's sum of P; lanes 32-63
-    // hold row 4 there, which stays zero, so halves_sum of register 0 gives
-    // the sum in both lanes of the query.
-    const half8 ones_a = ql == 0 ? (half8)E::round(1.0f) : (half8)(_Float16)0;
-    // V^T operand v (16-key step ks = v / MTX, output tile mt = v % MTX; the
-    // row-sum tile mt = MT takes the constant operand).
+    // A operand of the row sums (ROWSUM, a 16x16x32 MFMA with the 16-key P
+    // operand of 32 queries as B): the instruction takes lane l as column
+    // l % 16, contraction rows 8 (l / 16) .. +8, so lanes of even l / 16 bring
+    // queries 0-15, odd ones 16-31.  Row 0 has ones where l / 16 is even, row
+    // 4 where it is odd, the rest is zero: result register 0 holds query l's
+    // sum over the 16 keys in lane l < 32, zero in lanes 32-63.
+    const half8 ones_a =
+        gi == ((grp & 1) ? 4 : 0) ? (half8)E::round(1.0f) : (half8)(_Float16)0;
+    // V^T operand of P V slot v (16-key step ks = v / MTX, output tile mt = v % MTX;
+    // the row sums' slot mt = MT takes the constant operand).
     auto read_v = [&](const _Float16* Vs, int v) -> half8 {
       const int ks = v / MTX, mt = v % MTX;
       if (ROWSUM && mt == MT) return ones_a;
@@ -547,7 +553,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
     float16v oacc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) oacc[mt] = (float16v)0.0f;
-    float16v lacc = (float16v)0.0f;  // row-sum tile (ROWSUM)
+    float4v lacc = (float4v)0.0f;    // row sums (ROWSUM): register 0
     float m_run = -__builtin_inff();
     float l_run = 0.0f;              // the lane's part of its row sum (VALU row sums)
     const float c2 = a.c;  // |scale| * log2(e)
@@ -585,11 +591,12 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
                 float4{oacc[mt][4 * g], oacc[mt][4 * g + 1], oacc[mt][4 * g + 2],
                        oacc[mt][4 * g + 3]};
         pair_xo[MT * 1024 + lane] = m_run;
-        pair_xo[MT * 1024 + 64 + lane] = l_run;
+        pair_xo[MT * 1024 + 64 + lane] = ROWSUM ? lacc[0] : l_run;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) oacc[mt] = (float16v)0.0f;
         m_run = -__builtin_inff();
         l_run = 0.0f;
+        lacc = (float4v)0.0f;
         mc = 0.0f;
         thr = -__builtin_inff();
       }
@@ -779,7 +786,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
           constexpr int v = slot - PV_FIRST;
           constexpr int ks = v / MTX, mt = v % MTX;
           if constexpr (mt == MT)
-            lacc = E::mfma(vf[v], __builtin_bit_cast(half8, pf[ks]), lacc);
+            lacc = E::mfma16(vf[v], __builtin_bit_cast(half8, pf[ks]), lacc);
           else
             oacc[mt] = E::mfma(vf[v], __builtin_bit_cast(half8, pf[ks]), oacc[mt]);
         }
@@ -1051,28 +1058,33 @@ void launch_fused(const FwdArgs& a, int batch, bool causal, Schedule schedule,
 #define FA_LAUNCH(C, S, R, Y)                                                                 \
   hipLaunchKernelGGL((fa_fwd_kernel<D, C, S, WAVES, MASK, KSPLIT, BF16, R, Y>), grid, block, 0,   \
                      stream, args)
-  // Paired single-round launches at head_dim 64 take the ROWSUM instance
-  // (always static: pair_half is only set without counters).
-  if constexpr (D == 64 && WAVES == 4 && !MASK && !KSPLIT) {
-    if (causal && args.pair_half > 0) {
-      if (same) FA_LAUNCH(true, true, true, false); else FA_LAUNCH(true, false, true, false);
+  constexpr bool RS = D == 64;
+  // Non-causal launches without a mask: by rounds (see ROWSUM), counted in
+  // 128-row blocks for either workgroup shape, and none on the dynamic
+  // schedule, so that the kernels forced for a call give the same bits.
+  constexpr bool RS_FULL = RS && (MASK != 0 || KSPLIT);
+  if constexpr (RS && !RS_FULL) {
+    FwdArgs planned = a;
+    if (!dyn && !causal && plan_grid(planned, batch, 128) <= slots) {
+      if (same) FA_LAUNCH(false, true, RS, false); else FA_LAUNCH(false, false, RS, false);
       return;
     }
   }
   if constexpr (WAVES == 4) {
     if (dyn) {
       if (causal) {
-        if (same) FA_LAUNCH(true, true, false, true); else FA_LAUNCH(true, false, false, true);
+        if (same) FA_LAUNCH(true, true, RS, true); else FA_LAUNCH(true, false, RS, true);
       } else {
-        if (same) FA_LAUNCH(false, true, false, true); else FA_LAUNCH(false, false, false, true);
+        if (same) FA_LAUNCH(false, true, RS_FULL, true);
+        else FA_LAUNCH(false, false, RS_FULL, true);
       }
       return;
     }
   }
   if (causal) {
-    if (same) FA_LAUNCH(true, true, false, false); else FA_LAUNCH(true, false, false, false);
+    if (same) FA_LAUNCH(true, true, RS, false); else FA_LAUNCH(true, false, RS, false);
   } else {
-    if (same) FA_LAUNCH(false, true, false, false); else FA_LAUNCH(false, false, false, false);
+    if (same) FA_LAUNCH(false, true, RS_FULL, false); else FA_LAUNCH(false, false, RS_FULL, false);
   }
 #undef FA_LAUNCH
 }
