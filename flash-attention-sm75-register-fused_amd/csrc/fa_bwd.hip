@@ -113,9 +113,9 @@ int launch_backward(const BwdArgs& args, const BwdSplit& split, int batch, int h
   BwdArgs a = args;
   a.qtiles = (a.n + kBwdStatsTile - 1) / kBwdStatsTile;
   a.units = batch * (a.hq / a.group);
-  a.xcds = a.units % kNumXcds == 0 ? kNumXcds : 1;
   a.num_qblocks = (a.n + kBwdBlockRows - 1) / kBwdBlockRows;
   a.items = batch * a.hq * a.num_qblocks;
+  a.xcds = plan_xcds(a, a.units, a.items);
   a.pair_half = 0;
   a.mwords = (a.nk + 63) / 64;
   const bool mask = a.mbits != nullptr;

@@ -74,14 +74,33 @@ inline Schedule schedule_of_policy(int policy) {
   return policy == 3 ? Schedule::kDynamic : policy == 0 ? Schedule::kAuto : Schedule::kStatic;
 }
 
+// XCDs a call's units (u of them, `items` workgroups in all) are dealt to
+// whole.  With mask ranges per sequence the units of a padded batch hold very
+// different work (tiles outside a block's span are skipped), and an XCD that
+// holds the longest sequence's units sets the launch's time: such launches of
+// more than one workgroup per CU go out as one sequence, each unit's heads
+// over all XCDs, although K and V then pass through every L2.  Measured on
+// MI355X, bool causal masks with left padding of 0..3/8 N (us, units per XCD
+// against one sequence): forward B=4 Hq=14 Hkv=2 d64 N=2048 47.5 -> 39.9,
+// N=4096 159 -> 128, B=4 Hq=32 Hkv=8 N=2048 d128 161 -> 131, B=2 N=8192 866 ->
+// 856; backward B=2 Hq=32 Hkv=8 N=4096 d128 1222 -> 1089, B=8 H=8 N=2048 d64
+// 192 -> 177.  At one workgroup per CU or fewer the locality is worth more
+// (forward B=8 H=8 N=512 d64 12.0 against 12.5).  Order only: the same bits.
+template <class Args>
+inline int plan_xcds(const Args& a, int units, int64_t items) {
+  const bool uneven = a.mranges != nullptr && a.mrsb != 0;
+  if (units % kNumXcds != 0 || (uneven && items > resident_fused_workgroups() / 2)) return 1;
+  return kNumXcds;
+}
+
 // Fills num_qblocks, units, xcds and items of the fused kernel's work plan
 // for query blocks of block_m rows; returns the number of work items (the
 // grid size of the static schedule).
 inline int64_t plan_grid(FwdArgs& a, int batch, int block_m) {
   a.num_qblocks = (int)(((int64_t)a.n + block_m - 1) / block_m);
   a.units = batch * (a.hq / a.group);
-  a.xcds = a.units % kNumXcds == 0 ? kNumXcds : 1;
   a.items = batch * a.hq * a.num_qblocks;
+  a.xcds = plan_xcds(a, a.units, a.items);
   a.pair_half = 0;
   a.pair_split = 0;
   return a.items;

@@ -246,7 +246,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 //  * Workgroup wg runs on XCD wg % 8.  With a.xcds == 8 (units divisible by
 //    8) XCD x takes the units [x*U/8, (x+1)*U/8), so all query heads of a
 //    group, and all query blocks, that read one K/V pair share an L2.  With
-//    a.xcds == 1 the whole grid is one sequence.
+//    a.xcds == 1 the whole grid is one sequence (plan_xcds).
 //  * Within a sequence, workgroups go rank-major: rank r of every head before
 //    rank r+1.  Under causal masking rank 0 is the last (most expensive)
 //    query block, so the cheap blocks fill the tail of the launch.
