@@ -29,8 +29,8 @@
 //     per SIMD.
 // An explicit boolean mask (MASK instances) hides keys on top of the causal
 // rule; rows that see no key have lse = -inf, so their P is 0.
-// Tiles use the forward's LDS layout (Lds<D>: padded rows, 16-byte chunks
-// XOR-swizzled), on which both operand reads below are conflict-free.
+// Tiles use the forward's LDS layouts (BwdLds: 16-byte chunks XOR-swizzled),
+// on which both operand reads below are conflict-free.
 //
 // MFMA layouts (v_mfma_f32_32x32x16, as in fa_fwd_kernel.h):
 //   A[m][k]: lane l holds m = l%32, k = 8*(l/32) + j
@@ -54,50 +54,72 @@
 namespace fa {
 namespace {
 
-// Per-lane LDS addressing in one Lds<D> tile (64 rows):
+// LDS layout of the backward's tiles (64 rows of Q, dO, K or V): as the
+// forward's, dense rows at head_dim 64 (8 direct loads per tile where the
+// padded rows take 12), padded ones at 128.
+template <int D>
+using BwdLds = std::conditional_t<D == 64, LdsDense<64>, Lds<D == 64 ? 128 : D>>;
+
+// Per-lane LDS addressing in one tile:
 //   row(t, kk): the 8 columns 16kk + 8(l/32) .. +8 of row 32t + l%32 (an A
 //               or B operand whose m or n index is the tile row);
 //   tr(ks, mt): the A operand X^T of the row-major tile X: column 32mt + l%32
 //               of rows 16ks + {4(l/32) + 0..3, 8 + 4(l/32) + 0..3}, the
 //               order in which an accumulator's 16 rows arrive as B (two
 //               transposing ds_read_b64_tr_b16, 16 lanes = 4 rows x 16 columns).
+// Padded: the swizzle touches the low two chunk bits, so two bases each and
+// immediates for the rest; dense: a base per kk, and two per 32-column mt.
 template <int D>
 struct TileReader {
-  using L = Lds<D>;
-  int row_even, row_odd, tr0, tr1;
+  using L = BwdLds<D>;
+  static constexpr bool DENSE = D == 64;
+  int row_base[DENSE ? D / 16 : 2], tr0[DENSE ? D / 32 : 1], tr1[DENSE ? D / 32 : 1];
   __device__ __forceinline__ explicit TileReader(int lane) {
     const int hi = lane >> 5, ql = lane & 31, grp = lane >> 4, gi = lane & 15;
-    const int s = (ql >> 2) & 3;
-    row_even = ql * L::Pitch + 8 * (hi ^ s);
-    row_odd = ql * L::Pitch + 8 * ((2 + hi) ^ s);
     const int r = 4 * hi + (gi >> 2);
     const int c = 2 * (grp & 1) + ((gi & 3) >> 1);
-    tr0 = r * L::Pitch + 8 * (c ^ hi) + 4 * (gi & 1);
-    tr1 = (r + 8) * L::Pitch + 8 * (c ^ (hi + 2)) + 4 * (gi & 1);
+    if constexpr (DENSE) {
+#pragma unroll
+      for (int kk = 0; kk < D / 16; ++kk)
+        row_base[kk] = ql * L::Pitch + 8 * ((2 * kk + hi) ^ dense_swizzle(ql));
+#pragma unroll
+      for (int mt = 0; mt < D / 32; ++mt) {
+        tr0[mt] = r * L::Pitch + 8 * ((c + 4 * mt) ^ dense_swizzle(r)) + 4 * (gi & 1);
+        tr1[mt] = (r + 8) * L::Pitch + 8 * ((c + 4 * mt) ^ dense_swizzle(r + 8)) + 4 * (gi & 1);
+      }
+    } else {
+      const int s = (ql >> 2) & 3;
+      row_base[0] = ql * L::Pitch + 8 * (hi ^ s);
+      row_base[1] = ql * L::Pitch + 8 * ((2 + hi) ^ s);
+      tr0[0] = r * L::Pitch + 8 * (c ^ hi) + 4 * (gi & 1);
+      tr1[0] = (r + 8) * L::Pitch + 8 * (c ^ (hi + 2)) + 4 * (gi & 1);
+    }
   }
   __device__ __forceinline__ half8 row(const _Float16* tile, int t, int kk) const {
-    const int off = ((kk & 1) ? row_odd : row_even) + 32 * t * L::Pitch + 32 * (kk >> 1);
-    return *(const half8*)(tile + off);
+    if constexpr (DENSE) return *(const half8*)(tile + row_base[kk] + 32 * t * L::Pitch);
+    else
+      return *(const half8*)(tile + row_base[kk & 1] + 32 * t * L::Pitch + 32 * (kk >> 1));
   }
   __device__ __forceinline__ half8 tr(const _Float16* tile, int ks, int mt) const {
-    const int imm = 16 * ks * L::Pitch + 32 * mt;
-    const half4 lo = ds_read_tr16(tile + tr0 + imm);
-    const half4 hi4 = ds_read_tr16(tile + tr1 + imm);
+    const int imm = 16 * ks * L::Pitch + (DENSE ? 0 : 32 * mt);
+    const int m = DENSE ? mt : 0;
+    const half4 lo = ds_read_tr16(tile + tr0[m] + imm);
+    const half4 hi4 = ds_read_tr16(tile + tr1[m] + imm);
     return __builtin_shufflevector(lo, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
   }
 };
 
-// Global byte offset of lane `lane`'s 16 bytes in 1 KB segment `seg` of an
-// Lds<D> tile whose source rows are `stride` elements apart; -16 (past any
+// Global byte offset of lane `lane`'s 16 bytes in 1 KB segment `seg` of a
+// BwdLds<D> tile whose source rows are `stride` elements apart; -16 (past any
 // buffer window, so the lane writes zeros) for bytes in the row padding.
 template <int D>
 __device__ __forceinline__ int seg_offset(int seg, int lane, int64_t stride) {
-  using L = Lds<D>;
+  using L = BwdLds<D>;
   const int pos = seg * 1024 + 16 * lane;
   const int row = pos / (2 * L::Pitch);
   const int within = pos - row * (2 * L::Pitch);
   if (within >= 2 * D) return -16;
-  const int c = (within >> 4) ^ ((row >> 2) & 3);
+  const int c = (within >> 4) ^ (D == 64 ? dense_swizzle(row) : (row >> 2) & 3);
   return (int)(row * stride * 2) + 16 * c;
 }
 
@@ -144,7 +166,7 @@ __device__ __forceinline__ float* dkdv_part(const BwdSplit& sp, int slot, int ro
 template <int D, bool CAUSAL, bool MASK, bool BF16, class Split>
 __global__ void __launch_bounds__(512, 1) fa_bwd_dkdv_kernel(const BwdArgs a, const Split sp) {
   constexpr bool SPLIT = std::is_same<Split, BwdSplit>::value;
-  using L = Lds<D>;
+  using L = BwdLds<D>;
   using E = Elem<BF16>;
   constexpr int KK = D / 16;
   constexpr int MT = D / 32;
@@ -683,7 +705,7 @@ __global__ void __launch_bounds__(256) fa_bwd_merge_kernel(const BwdArgs a, cons
 // block masks run in a loop of their own, free of mask code.
 template <int D, bool CAUSAL, bool MASK, bool BF16>
 __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kernel(const BwdArgs a) {
-  using L = Lds<D>;
+  using L = BwdLds<D>;
   using E = Elem<BF16>;
   constexpr int KK = D / 16;
   constexpr int MT = D / 32;
@@ -836,6 +858,10 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
     const uint64_t mw = MASK ? mrow[j] : ~0ull;
     bool need_mask = kstart + kBlockN > NK || (CAUSAL && kstart + kBlockN - 1 > qw + a.diag);
     if (MASK) need_mask = need_mask || __builtin_amdgcn_ballot_w64(~mw != 0) != 0;
+    // Bit 8 (i / 4) + i % 4 of mws[t]: element (t, i).  The halves are shifted
+    // apart: a 64-bit shift by a lane's amount misreads an amount in the last
+    // of 256 registers.
+    const uint32_t mws[2] = {(uint32_t)mw >> (4 * hi), (uint32_t)(mw >> 32) >> (4 * hi)};
     uint4v pd[4];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -850,10 +876,12 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
         float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i], c2, -lse2));
         float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i + 1], c2, -lse2));
         if (MASKED && need_mask) {
-          const int kt = 32 * t + 8 * (i >> 2) + 4 * hi + (i & 3);  // key within the tile
-          const int key = kstart + kt;
-          if (key >= NK || (CAUSAL && key > qrow + a.diag) || ((mw >> kt) & 1) == 0) p0 = 0.0f;
-          if (key + 1 >= NK || (CAUSAL && key + 1 > qrow + a.diag) || ((mw >> (kt + 1)) & 1) == 0)
+          const int off = 8 * (i >> 2) + (i & 3);
+          const int key = kstart + 32 * t + off + 4 * hi;
+          if (key >= NK || (CAUSAL && key > qrow + a.diag) || (MASK && ((mws[t] >> off) & 1) == 0))
+            p0 = 0.0f;
+          if (key + 1 >= NK || (CAUSAL && key + 1 > qrow + a.diag) ||
+              (MASK && ((mws[t] >> (off + 1)) & 1) == 0))
             p1 = 0.0f;
         }
         put_pair<E>(pd, t, i, p0 * dpa[i], p1 * dpa[i + 1]);

@@ -622,7 +622,10 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
           (kstart + kBlockN > NK) || (CAUSAL && kstart + kBlockN - 1 > qw_j + a.diag);
       if (MASK) need_mask = need_mask || __builtin_amdgcn_ballot_w64(~mw != 0) != 0;
       if (need_mask) {
-        const uint64_t mws = mw >> (4 * hi);  // bit 32 t + 8 (i / 4) + i % 4: element (t, i)
+        // Bit 8 (i / 4) + i % 4 of mws[t]: element (t, i).  The halves are shifted
+        // apart: a 64-bit shift by a lane's amount misreads an amount in the
+        // last of 256 registers.
+        const uint32_t mws[2] = {(uint32_t)mw >> (4 * hi), (uint32_t)(mw >> 32) >> (4 * hi)};
         // Element (t, i) holds key kstart + 4 hi + off, off = 32 t + 8 (i / 4)
         // + i % 4 (a constant); it is visible iff off <= lim.
         const int last = CAUSAL ? min(NK - 1, qrow_j + a.diag) : NK - 1;
@@ -634,7 +637,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
           constexpr int t = e >> 4, i = e & 15;
           constexpr int off = 32 * t + 8 * (i >> 2) + (i & 3);
           bool masked = off > lim;
-          if (MASK) masked = masked || ((mws >> off) & 1) == 0;
+          if (MASK) masked = masked || ((mws[t] >> (off & 31)) & 1) == 0;
           if (masked) s[t][i] = -__builtin_inff();
         });
         mx = row_max(s);
