@@ -714,6 +714,8 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
   __shared__ __attribute__((aligned(1024))) _Float16 k_lds1[L::Tile];
   __shared__ __attribute__((aligned(1024))) _Float16 v_lds0[L::Tile];
   __shared__ __attribute__((aligned(1024))) _Float16 v_lds1[L::Tile];
+  __shared__ __attribute__((aligned(1024))) _Float16 k_lds2[D == 64 ? L::Tile : 1];
+  __shared__ __attribute__((aligned(1024))) _Float16 v_lds2[D == 64 ? L::Tile : 1];
 
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = (int)threadIdx.x & 63;
@@ -843,83 +845,261 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
   const TileReader<D> rd(lane);
   const float c2 = a.c2;
 
-  // One key tile j on buffer parity PAR.  MASKED: the tile may need the
-  // per-element mask (tested per pair, on this wave's need_mask); the
-  // unmasked tiles run without any mask code, so the compiler interleaves
-  // their exps with the MFMAs (a branch per pair splits the tile into blocks).
-  auto step = [&](int j, auto par_t, auto masked_t) {
-    constexpr int PAR = decltype(par_t)::value;
-    constexpr bool MASKED = decltype(masked_t)::value;
-    const _Float16* kc = PAR ? k_lds1 : k_lds0;
-    const _Float16* vc = PAR ? v_lds1 : v_lds0;
-    if (j + 1 < ntiles) issue(j + 1, PAR ? k_lds0 : k_lds1, PAR ? v_lds0 : v_lds1);
-    const int kstart = j * kBlockN;
-    // MASK: bit k of mw = key kstart + k visible to this lane's query.
-    const uint64_t mw = MASK ? mrow[j] : ~0ull;
-    bool need_mask = kstart + kBlockN > NK || (CAUSAL && kstart + kBlockN - 1 > qw + a.diag);
-    if (MASK) need_mask = need_mask || __builtin_amdgcn_ballot_w64(~mw != 0) != 0;
-    // Bit 8 (i / 4) + i % 4 of mws[t]: element (t, i).  The halves are shifted
-    // apart: a 64-bit shift by a lane's amount misreads an amount in the last
-    // of 256 registers.
-    const uint32_t mws[2] = {(uint32_t)mw >> (4 * hi), (uint32_t)(mw >> 32) >> (4 * hi)};
-    uint4v pd[4];
+  if constexpr (D == 64) {
+    // Head_dim 64: software pipelined over 32-key sub-tiles and hand ordered, as
+    // the forward.  Step (j, t) issues the MFMAs of S and dP of the next
+    // sub-tile, alternating, then dQ's of (j, t), and each slot carries the LDS
+    // reads of three slots ahead and a share of (j, t)'s element work (P, dS);
+    // left to the compiler, the element work of a sub-tile sat between its own
+    // products with the matrix pipe idle.  The scores' accumulators of two
+    // sub-tiles fit two workgroups per CU at this head_dim only.  K and V tiles
+    // are triple buffered: tile j's steps read tiles j and j + 1 and load
+    // j + 2; one barrier per tile.
+    const float c2n = c2 != 0.0f ? c2 : 1e-30f;  // hidden scores: +-inf, so P is 0
+    const float mval = c2n > 0.0f ? -__builtin_inff() : __builtin_inff();
+    auto kbuf = [&](auto st) -> _Float16* {
+      constexpr int S = decltype(st)::value % 3;
+      if constexpr (S == 0) return k_lds0;
+      else if constexpr (S == 1) return k_lds1;
+      else return k_lds2;
+    };
+    auto vbuf = [&](auto st) -> _Float16* {
+      constexpr int S = decltype(st)::value % 3;
+      if constexpr (S == 0) return v_lds0;
+      else if constexpr (S == 1) return v_lds1;
+      else return v_lds2;
+    };
+    auto window = [&](const _Float16* base, int64_t stride, int j) {
+      const int rows = NK - j * kBlockN;
+      return make_rsrc(base + (int64_t)j * kBlockN * stride, rows > 0 ? (int)(rows * stride * 2) : 0);
+    };
+    auto load_tile = [&](int j, auto st) {
+      const __amdgpu_buffer_rsrc_t rk = window(Kp, a.ksn, j), rv = window(Vp, a.vsn, j);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float16v sa = (float16v)0.0f, dpa = ndv;
+      for (int q = 0; q < SEGQ; ++q)
+        direct_load16(rk, (lds_void*)(kbuf(st) + (wave + 4 * q) * 512), goff_k[q]);
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) sa = E::mfma(rd.row(kc, t, kk), qf[kk], sa);
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) dpa = E::mfma(rd.row(vc, t, kk), df[kk], dpa);
-      // Element i: key kstart + 32t + 8(i/4) + 4hi + i%4, query qrow.
-#pragma unroll
-      for (int i = 0; i < 16; i += 2) {
-        float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i], c2, -lse2));
-        float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i + 1], c2, -lse2));
-        if (MASKED && need_mask) {
-          const int off = 8 * (i >> 2) + (i & 3);
-          const int key = kstart + 32 * t + off + 4 * hi;
-          if (key >= NK || (CAUSAL && key > qrow + a.diag) || (MASK && ((mws[t] >> off) & 1) == 0))
-            p0 = 0.0f;
-          if (key + 1 >= NK || (CAUSAL && key + 1 > qrow + a.diag) ||
-              (MASK && ((mws[t] >> (off + 1)) & 1) == 0))
-            p1 = 0.0f;
+      for (int q = 0; q < SEGQ; ++q)
+        direct_load16(rv, (lds_void*)(vbuf(st) + (wave + 4 * q) * 512), goff_v[q]);
+    };
+    float16v sb[2], db[2];  // S and dP of the sub-tile of parity t in flight
+    uint64_t mw = ~0ull;    // MASK: the lane's mask word of the current tile
+    // Hidden scores of sub-tile (j, t) to mval, where the tile crosses the
+    // keys' end, the wave's diagonal or the mask.
+    auto prepare = [&](int j, auto t_c, uint64_t word) {
+      constexpr int t = decltype(t_c)::value;
+      const int k0 = j * kBlockN + 32 * t;
+      const uint32_t wt = (uint32_t)(word >> (32 * t));
+      bool need = k0 + 32 > NK || (CAUSAL && k0 + 31 > qw + a.diag);
+      if (MASK) need = need || __builtin_amdgcn_ballot_w64(~wt != 0) != 0;
+      if (need) {
+        const int lim = (CAUSAL ? min(NK - 1, qrow + a.diag) : NK - 1) - k0 - 4 * hi;
+        const uint32_t bits = wt >> (4 * hi);
+        static_for<16>([&](auto i_c) {
+          constexpr int i = decltype(i_c)::value;
+          constexpr int off = 8 * (i >> 2) + (i & 3);
+          if (off > lim || (MASK && ((bits >> off) & 1) == 0)) sb[t][i] = mval;
+        });
+      }
+    };
+    // Step (j, t), tile j at position U of the unrolled loop.  NEXT: tile j + 1
+    // exists.
+    auto step = [&](int j, auto u_c, auto t_c, auto next_c) {
+      constexpr int U = decltype(u_c)::value;
+      constexpr int t = decltype(t_c)::value;
+      constexpr bool NEXT = decltype(next_c)::value;
+      constexpr bool HAS = t == 0 || NEXT;      // another sub-tile follows
+      constexpr int NSD = HAS ? 2 * KK : 0;     // S and dP MFMAs
+      constexpr int NSLOT = NSD + 2 * MT;       // then dQ's
+      constexpr int PF = 3;                     // operand reads run this many slots ahead
+      constexpr int tn = 1 - t;
+      const _Float16* kn = kbuf(std::integral_constant<int, U + t>{});  // the next sub-tile's
+      const _Float16* vn = vbuf(std::integral_constant<int, U + t>{});
+      const _Float16* kc = kbuf(u_c);
+      uint64_t mw_next = ~0ull;
+      __amdgpu_buffer_rsrc_t rk, rv;
+      if constexpr (t == 0 && NEXT) {
+        if (MASK) mw_next = mrow[j + 1];
+        rk = window(Kp, a.ksn, j + 2);
+        rv = window(Vp, a.vsn, j + 2);
+      }
+      auto operand = [&](int slot) -> half8 {
+        if (slot < NSD)
+          return (slot & 1) ? rd.row(vn, tn, slot >> 1) : rd.row(kn, tn, slot >> 1);
+        return rd.tr(kc, 2 * t + (slot - NSD) / MT, (slot - NSD) % MT);
+      };
+      uint4v pd[2];
+      auto pair = [&](int pr) {
+        const int i = 2 * pr;
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sb[t][i], c2n, -lse2));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sb[t][i + 1], c2n, -lse2));
+        unsigned x = __builtin_bit_cast(unsigned, E::pack(p0 * db[t][i], p1 * db[t][i + 1]));
+        asm volatile("" : "+v"(x));  // keeps the pair in its slot
+        pd[i >> 3][(i & 7) >> 1] = x;
+      };
+      // Pairs 0-3 precede the first dQ MFMA, 4-7 the third.
+      constexpr auto pair_slot = [](int pr) constexpr {
+        if (NSD == 0) return pr < 4 ? -1 : (pr - 4) / 2;
+        const int spread = (pr * (NSD + MT)) / 8, last = pr < 4 ? NSD - 1 : NSD + MT - 1;
+        return spread < last ? spread : last;
+      };
+      half8 op[NSLOT];
+      static_for<PF>([&](auto i_c) { op[decltype(i_c)::value] = operand(decltype(i_c)::value); });
+      static_for<8>([&](auto p_c) {
+        if constexpr (pair_slot(decltype(p_c)::value) < 0) pair(decltype(p_c)::value);
+      });
+      static_for<NSLOT>([&](auto slot_c) {
+        constexpr int slot = decltype(slot_c)::value;
+        if constexpr (slot + PF < NSLOT) op[slot + PF] = operand(slot + PF);
+        if constexpr (slot < NSD) {
+          constexpr int kk = slot >> 1;
+          if constexpr (slot & 1) db[tn] = E::mfma(op[slot], df[kk], kk == 0 ? ndv : db[tn]);
+          else sb[tn] = E::mfma(op[slot], qf[kk], kk == 0 ? (float16v)0.0f : sb[tn]);
+        } else {
+          constexpr int v = slot - NSD;
+          dq[v % MT] = E::mfma(op[slot], __builtin_bit_cast(half8, pd[v / MT]), dq[v % MT]);
         }
-        put_pair<E>(pd, t, i, p0 * dpa[i], p1 * dpa[i + 1]);
+        if constexpr (t == 0 && NEXT && slot % 2 == 0 && slot / 2 < 2 * SEGQ) {
+          constexpr int q = slot / 2;
+          if constexpr (q < SEGQ)
+            direct_load16(rk, (lds_void*)(kbuf(std::integral_constant<int, U + 2>{}) + (wave + 4 * q) * 512),
+                          goff_k[q]);
+          else
+            direct_load16(rv, (lds_void*)(vbuf(std::integral_constant<int, U + 2>{}) +
+                                          (wave + 4 * (q - SEGQ)) * 512),
+                          goff_v[q - SEGQ]);
+        }
+        static_for<8>([&](auto p_c) {
+          if constexpr (pair_slot(decltype(p_c)::value) == slot) pair(decltype(p_c)::value);
+        });
+        fence_schedule();
+      });
+      if constexpr (t == 0) {
+        prepare(j, std::integral_constant<int, 1>{}, mw);
+        if constexpr (NEXT) mw = mw_next;
+      } else if constexpr (NEXT) {
+        prepare(j + 1, std::integral_constant<int, 0>{}, mw);
+        barrier_after_loads<0>();
+      }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    auto tile = [&](int j, auto u_c, auto next_c) {
+      step(j, u_c, I0{}, next_c);
+      step(j, u_c, I1{}, next_c);
+    };
+    if (ntiles > j_begin) {
+      load_tile(j_begin, I0{});
+      load_tile(j_begin + 1, I1{});  // (zeros past the keys)
+      if (MASK) mw = mrow[j_begin];
+      barrier_after_loads<2 * SEGQ + (MASK ? 1 : 0)>();  // the first tile has landed
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        sb[0] = E::mfma(rd.row(k_lds0, 0, kk), qf[kk], kk == 0 ? (float16v)0.0f : sb[0]);
+        db[0] = E::mfma(rd.row(v_lds0, 0, kk), df[kk], kk == 0 ? ndv : db[0]);
+      }
+      prepare(j_begin, I0{}, mw);
+      barrier_after_loads<0>();
+      int j = j_begin;
+      for (; j + 3 < ntiles; j += 3) {
+        tile(j, I0{}, Flag<true>{});
+        tile(j + 1, I1{}, Flag<true>{});
+        tile(j + 2, I2{}, Flag<true>{});
+      }
+      const int rest = ntiles - j;  // 1 .. 3
+      if (rest == 1) {
+        tile(j, I0{}, Flag<false>{});
+      } else if (rest == 2) {
+        tile(j, I0{}, Flag<true>{});
+        tile(j + 1, I1{}, Flag<false>{});
+      } else {
+        tile(j, I0{}, Flag<true>{});
+        tile(j + 1, I1{}, Flag<true>{});
+        tile(j + 2, I2{}, Flag<false>{});
       }
     }
+    // No direct load may land in LDS after the workgroup ends.
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+  } else {
+    // One key tile j on buffer parity PAR.  MASKED: the tile may need the
+    // per-element mask (tested per pair, on this wave's need_mask); the
+    // unmasked tiles run without any mask code, so the compiler interleaves
+    // their exps with the MFMAs (a branch per pair splits the tile into blocks).
+    auto step = [&](int j, auto par_t, auto masked_t) {
+      constexpr int PAR = decltype(par_t)::value;
+      constexpr bool MASKED = decltype(masked_t)::value;
+      const _Float16* kc = PAR ? k_lds1 : k_lds0;
+      const _Float16* vc = PAR ? v_lds1 : v_lds0;
+      if (j + 1 < ntiles) issue(j + 1, PAR ? k_lds0 : k_lds1, PAR ? v_lds0 : v_lds1);
+      const int kstart = j * kBlockN;
+      // MASK: bit k of mw = key kstart + k visible to this lane's query.
+      const uint64_t mw = MASK ? mrow[j] : ~0ull;
+      bool need_mask = kstart + kBlockN > NK || (CAUSAL && kstart + kBlockN - 1 > qw + a.diag);
+      if (MASK) need_mask = need_mask || __builtin_amdgcn_ballot_w64(~mw != 0) != 0;
+      // Bit 8 (i / 4) + i % 4 of mws[t]: element (t, i).  The halves are shifted
+      // apart: a 64-bit shift by a lane's amount misreads an amount in the last
+      // of 256 registers.
+      const uint32_t mws[2] = {(uint32_t)mw >> (4 * hi), (uint32_t)(mw >> 32) >> (4 * hi)};
+      uint4v pd[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+      for (int t = 0; t < 2; ++t) {
+        float16v sa = (float16v)0.0f, dpa = ndv;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        dq[mt] = E::mfma(rd.tr(kc, ks, mt), __builtin_bit_cast(half8, pd[ks]), dq[mt]);
-    }
-    barrier_after_loads<0>();
-  };
+        for (int kk = 0; kk < KK; ++kk) sa = E::mfma(rd.row(kc, t, kk), qf[kk], sa);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) dpa = E::mfma(rd.row(vc, t, kk), df[kk], dpa);
+        // Element i: key kstart + 32t + 8(i/4) + 4hi + i%4, query qrow.
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+          float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i], c2, -lse2));
+          float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i + 1], c2, -lse2));
+          if (MASKED && need_mask) {
+            const int off = 8 * (i >> 2) + (i & 3);
+            const int key = kstart + 32 * t + off + 4 * hi;
+            if (key >= NK || (CAUSAL && key > qrow + a.diag) || (MASK && ((mws[t] >> off) & 1) == 0))
+              p0 = 0.0f;
+            if (key + 1 >= NK || (CAUSAL && key + 1 > qrow + a.diag) ||
+                (MASK && ((mws[t] >> (off + 1)) & 1) == 0))
+              p1 = 0.0f;
+          }
+          put_pair<E>(pd, t, i, p0 * dpa[i], p1 * dpa[i + 1]);
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          dq[mt] = E::mfma(rd.tr(kc, ks, mt), __builtin_bit_cast(half8, pd[ks]), dq[mt]);
+      }
+      barrier_after_loads<0>();
+    };
 
-  // Tiles [0, j_split) need no mask for any wave of the workgroup (wave 0,
-  // whose rows come first, is the first to meet its diagonal; every tile
-  // lies inside the keys); the rest run the masked step.  With a boolean mask
-  // any tile may need it.
-  int j_split = 0;
-  if (!MASK) {
-    j_split = min(ntiles, NK / kBlockN);
-    if (CAUSAL) j_split = min(j_split, max(0, q0 + a.diag + 1) / kBlockN);
-  }
-  using P0 = std::integral_constant<int, 0>;
-  using P1 = std::integral_constant<int, 1>;
-  // Tile j sits in the buffers of parity j & 1.
-  if (ntiles > j_begin)
-    issue(j_begin, (j_begin & 1) ? k_lds1 : k_lds0, (j_begin & 1) ? v_lds1 : v_lds0);
-  barrier_after_loads<0>();
-  int j = j_begin;
-  for (; j + 1 < j_split; j += 2) {
-    step(j, P0{}, Flag<false>{});
-    step(j + 1, P1{}, Flag<false>{});
-  }
-  if (j < j_split) step(j++, P0{}, Flag<false>{});
-  for (; j < ntiles; ++j) {
-    if (j & 1) step(j, P1{}, Flag<true>{});
-    else step(j, P0{}, Flag<true>{});
+    // Tiles [0, j_split) need no mask for any wave of the workgroup (wave 0,
+    // whose rows come first, is the first to meet its diagonal; every tile
+    // lies inside the keys); the rest run the masked step.  With a boolean mask
+    // any tile may need it.
+    int j_split = 0;
+    if (!MASK) {
+      j_split = min(ntiles, NK / kBlockN);
+      if (CAUSAL) j_split = min(j_split, max(0, q0 + a.diag + 1) / kBlockN);
+    }
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    // Tile j sits in the buffers of parity j & 1.
+    if (ntiles > j_begin)
+      issue(j_begin, (j_begin & 1) ? k_lds1 : k_lds0, (j_begin & 1) ? v_lds1 : v_lds0);
+    barrier_after_loads<0>();
+    int j = j_begin;
+    for (; j + 1 < j_split; j += 2) {
+      step(j, P0{}, Flag<false>{});
+      step(j + 1, P1{}, Flag<false>{});
+    }
+    if (j < j_split) step(j++, P0{}, Flag<false>{});
+    for (; j < ntiles; ++j) {
+      if (j & 1) step(j, P1{}, Flag<true>{});
+      else step(j, P0{}, Flag<true>{});
+    }
   }
 
   if (qrow < N) {
