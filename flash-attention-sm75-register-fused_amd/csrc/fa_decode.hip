@@ -99,6 +99,13 @@ constexpr int kMergeLoads = 8;
 // combine kernels' many (Hq=32 Hkv=8 8 rows 2048 keys d128, 128 KB: 14.8 us
 // merged here, 11.1 by the combine kernel; 64 KB within 0.7 us either way).
 constexpr int kMergeMaxBytes = 64 << 10;
+// ... and at head_dim 64 not where many units of many splits fill the GPU:
+// every CU then ends with a merge of short partials, which the next launch
+// cannot overlap (B=2 Hq=8 Hkv=8 4096 keys d64, 16 units of 16 splits: 9.5
+// merged here, 8.8 by the combine kernel; B=16 H=1 16384 keys 16.9 and 16.1;
+// 8 splits, B=4 H=8 4096 keys, 11.5 and 11.6).
+constexpr int kMergeMaxSplits64 = 8;
+constexpr int kMergeFewWgs = 128;
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1017,7 +1024,9 @@ DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
   pl.chunk_tiles = std::max(1, (pl.tiles + splits - 1) / splits);
   pl.splits = std::max(1, (pl.tiles + pl.chunk_tiles - 1) / pl.chunk_tiles);
   pl.merge_in_kernel = pl.splits > 1 && pl.splits <= kThreads &&
-                       (int64_t)pl.splits * pl.rows * head_dim * 4 <= kMergeMaxBytes;
+                       (int64_t)pl.splits * pl.rows * head_dim * 4 <= kMergeMaxBytes &&
+                       (head_dim != 64 || pl.splits <= kMergeMaxSplits64 ||
+                        (int64_t)pl.units * pl.splits <= kMergeFewWgs);
   pl.workspace_bytes = 0;
   if (pl.splits > 1) {
     // Partials, then the marks in whole records of one split (a size of that
