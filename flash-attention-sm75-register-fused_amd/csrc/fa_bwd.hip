@@ -27,11 +27,14 @@ namespace fa {
 // N=2048 d128 full 500 -> 418 us.  Where the unsplit launch already fills the
 // GPU a split loses (B=1 Hq=32 Hkv=8 N=8192 d128 causal 1605 -> 1658-1790 us,
 // B=4 H=8 N=2048 d64 causal 85 -> 95-112 us, B=4 H=12 N=1024 d64 full 69 -> 80
-// us): it must be estimated kMinGain faster to be taken.
+// us): it must be estimated kMinGain faster to be taken, and to save kMinSaved
+// steps (about a microsecond each), since the merge launch costs the host 3 us
+// (B=1 H=12 N=1114 d64 full, 4 steps saved: 40.3 us unsplit, 42.0 split).
 constexpr int kPieceSteps = 8;
 constexpr int kMergeSteps = 5;
 constexpr int kMinPiece = 8;  // shortest T considered (T = 4 on the N=1024 shape below: 45 us)
 constexpr double kMinGain = 1.08;
+constexpr int kMinSaved = 8;
 constexpr int kMaxPiecesPerCu = 4;  // bounds the partials: 134 MB at head_dim 128 on 256 CUs
 
 int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, BwdSplit& s) {
@@ -43,6 +46,9 @@ int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, B
   const int64_t units = (int64_t)batch * (a.hq / a.group);
   const int cus = resident_fused_workgroups() / 2;
   const int64_t qtiles = ((int64_t)a.n + kBwdStatsTile - 1) / kBwdStatsTile;
+  // Equal blocks run in whole rounds; under a mask their steps are an upper
+  // bound and the rounds are not whole (B=1 H=8 N=6016 d128, causal mask: 376
+  // blocks split for their rounds 467 us, unsplit 426).
   int64_t steps[kBwdMaxSplitBlocks], longest = 0, shortest = INT64_MAX, sum = 0;
   for (int kb = 0; kb < nkb; ++kb) {
     const int64_t q_first =
@@ -54,12 +60,13 @@ int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, B
     shortest = std::min(shortest, steps[kb]);
     sum += steps[kb];
   }
+  const bool equal = longest == shortest && a.mbits == nullptr;
   const double load = (double)sum * units / cus;  // steps per CU
   // No split can be estimated below a CU's mean load: most launches that fill
   // the GPU end here.
   const int64_t rounds = (nkb * units + cus - 1) / cus;
   const double one_each =
-      longest == shortest
+      equal
           ? (double)((longest + kPieceSteps) * rounds)
           : std::max((double)longest + kPieceSteps, load + (double)kPieceSteps * nkb * units / cus);
   if ((std::max(load, (double)kMinPiece) + kPieceSteps + kMergeSteps) * kMinGain > one_each)
@@ -76,7 +83,7 @@ int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, B
     if (count > kBwdMaxPieces || total > (int64_t)kMaxPiecesPerCu * cus) break;
     double est = (double)t + kPieceSteps;
     if (total > cus) {
-      if (longest == shortest)
+      if (equal)
         est *= (double)((total + cus - 1) / cus);
       else
         est = std::max(est, load + (double)kPieceSteps * total / cus +
@@ -87,7 +94,7 @@ int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, B
       best_t = t;
     }
   }
-  if (best_t == 0 || best * kMinGain > one_each) return 0;
+  if (best_t == 0 || best * kMinGain > one_each || best + kMinSaved > one_each) return 0;
   int64_t n[kBwdMaxSplitBlocks];
   int first = 0;
   for (int kb = 0; kb < nkb; ++kb) {

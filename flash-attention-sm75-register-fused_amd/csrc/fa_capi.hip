@@ -362,6 +362,7 @@ int64_t bwd_split(const fa_bwd_params* p, fa::BwdSplit& split) {
   a.diag = p->causal == FA_CAUSAL_BOTTOM_RIGHT ? a.nk - a.n : 0;
   a.hq = (int)p->heads_q;
   a.group = (int)(p->heads_q / p->heads_kv);
+  a.mbits = reinterpret_cast<const uint64_t*>(p->mask_bits);
   return fa::plan_bwd_split(a, (int)p->batch, (int)p->head_dim, p->causal != FA_CAUSAL_NONE, split);
 }
 

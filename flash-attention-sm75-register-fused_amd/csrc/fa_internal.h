@@ -74,7 +74,7 @@ inline Schedule schedule_of_policy(int policy) {
   return policy == 3 ? Schedule::kDynamic : policy == 0 ? Schedule::kAuto : Schedule::kStatic;
 }
 
-// XCDs a call's units (u of them, `items` workgroups in all) are dealt to
+// XCDs a call's units (`units` of them, `items` workgroups in all) are dealt to
 // whole.  With mask ranges per sequence the units of a padded batch hold very
 // different work (tiles outside a block's span are skipped), and an XCD that
 // holds the longest sequence's units sets the launch's time: such launches of
@@ -85,10 +85,12 @@ inline Schedule schedule_of_policy(int policy) {
 // N=4096 159 -> 128, B=4 Hq=32 Hkv=8 N=2048 d128 161 -> 131, B=2 N=8192 866 ->
 // 856; backward B=2 Hq=32 Hkv=8 N=4096 d128 1222 -> 1089, B=8 H=8 N=2048 d64
 // 192 -> 177.  At one workgroup per CU or fewer the locality is worth more
-// (forward B=8 H=8 N=512 d64 12.0 against 12.5).  Order only: the same bits.
+// (forward B=8 H=8 N=512 d64 12.0 against 12.5), and so it is for one sequence,
+// whose heads hold equal work.  Order only: the same bits.
 template <class Args>
 inline int plan_xcds(const Args& a, int units, int64_t items) {
-  const bool uneven = a.mranges != nullptr && a.mrsb != 0;
+  const int sequences = units / (a.hq / a.group);
+  const bool uneven = a.mranges != nullptr && a.mrsb != 0 && sequences > 1;
   if (units % kNumXcds != 0 || (uneven && items > resident_fused_workgroups() / 2)) return 1;
   return kNumXcds;
 }

@@ -10,7 +10,7 @@ import pytest
 from capi_types import LIB, BwdParams
 
 
-def partials(B, Hq, Hkv, Nq, Nk, D, causal):
+def partials(B, Hq, Hkv, Nq, Nk, D, causal, mask=False):
     """(bytes beyond the required part, bytes of one piece's partials)"""
     if not os.path.exists(LIB):
         pytest.fail(f"{LIB} not built: run __graft_entry__.build()")
@@ -19,6 +19,7 @@ def partials(B, Hq, Hkv, Nq, Nk, D, causal):
     p = BwdParams()
     p.batch, p.heads_q, p.heads_kv, p.seq_len, p.seq_len_kv, p.head_dim, p.causal = (
         B, Hq, Hkv, Nq, Nk, D, causal)
+    p.mask_bits = 256 if mask else None  # only tested for null
     need = B * Hq * ((Nq + 63) // 64) * 520
     extra = f(ctypes.byref(p)) - need
     assert extra >= 0
@@ -31,6 +32,10 @@ def partials(B, Hq, Hkv, Nq, Nk, D, causal):
     ((1, 32, 8, 8192, 8192, 128, 1), False), ((4, 8, 8, 2048, 2048, 64, 1), False),
     ((4, 12, 12, 1024, 1024, 64, 0), False), ((2, 8, 2, 100, 100, 128, 0), False),
     ((1, 64, 1, 64, 40000, 64, 0), False),          # more key blocks than the tables hold
+    ((1, 12, 12, 1114, 1114, 64, 0), False),        # saves less than the merge launch costs
+    ((1, 8, 8, 6016, 6016, 128, 0), True),          # two whole rounds of equal blocks ...
+    ((1, 8, 8, 6016, 6016, 128, 0, True), False),   # ... which a mask makes uneven
+    ((4, 16, 4, 448, 448, 128, 0, True), True),
 ])
 def test_which_calls_split(call, split):
     assert (partials(*call)[0] > 0) == split
