@@ -98,7 +98,8 @@ namespace {
 // Hq=14 Hkv=2 N=1777 causal 27.3 / 28.2, B=1 Hq=32 Hkv=8 N=8192 causal 303 /
 // 312, B=2 Hq=64 Hkv=8 N=16384 causal 4593 / 4756, B=2 H=8 N=4096 full, one
 // round, 75.2 / 77.2; but B=2 H=24 N=1500 full 44.2 / 42.2, B=8 H=16 N=1024
-// full 44.9 / 43.5).
+// full 44.9 / 43.5).  A wave whose P are not all finite sums them again after
+// the loop (sum_again).
 // DYN: the instance carries the dynamic schedule's item loop (4-wave launches
 // that run it).  Static launches take instances without it: the loop's
 // claim, prefetch and hand-off state costs registers all through the steps
@@ -946,8 +947,93 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
     // No direct load may land in LDS after the workgroup ends.
     __builtin_amdgcn_s_waitcnt(0x0F70);
     // From here on l_run is the lane's part of its row sum either way (the
-    // row-sum tile holds all of it in lanes 0-31, zero in lanes 32-63).
-    if constexpr (ROWSUM) l_run = lacc[0];
+    // row-sum MFMAs hold all of it in lanes 0-31, zero in lanes 32-63).
+    if constexpr (ROWSUM) {
+      // Those MFMAs contract the P of queries c and c + 16 together, the other
+      // query's against zeros: where one of the two has a P that is no finite
+      // number the product is NaN and takes the other's sum with it.  Lanes
+      // 32-63, whose rows are all zeros, show it.  Such a wave sums again,
+      // outside the loop, which keeps its rate; the sum is of the same rounded P
+      // (relative to the final running max), the lane's half of each row.
+      // It reads its parameters again, through a pointer the compiler does not
+      // know: kept in registers over the loop they spilled scalars there.
+      auto sum_again = [&](int row, int t0, int t1, float m) -> float {
+        const __attribute__((address_space(4))) FwdArgs* p =
+            (const __attribute__((address_space(4))) FwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        const float c = p->c;
+        const float off = (m == -__builtin_inff()) ? 0.0f : m * c;
+        const int keys = p->nk;
+        const int last = CAUSAL ? min(keys - 1, row + p->diag) : keys - 1;
+        const int rq = min(row, p->n - 1);
+        const _Float16* qp = p->q + b * p->qsb + hq * p->qsh + (int64_t)rq * p->qsn + 8 * hi;
+        const _Float16* k0 = p->k + b * p->ksb + hq / p->group * p->ksh + 8 * hi;
+        half8 qr[KK];
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+          qr[kk] = *(const half8*)(qp + 16 * kk);
+          if (p->negate_q) qr[kk] = negate16(qr[kk]);
+        }
+        float sum = 0.0f;
+        for (int j = t0; j < t1; ++j) {
+          uint64_t word = ~0ull;
+          if constexpr (KEY_BYTES) {
+            const uint8_t* kb = p->mkeys + b * p->mksb;
+            word = __builtin_amdgcn_ballot_w64(
+                kb[(int64_t)min(j * kBlockN + lane, keys - 1) * p->mksk] != 0);
+          } else if constexpr (MASK) {
+            word = p->mbits[b * p->msb + hq * p->msh + (int64_t)rq * p->msq + j];
+          }
+#pragma unroll 1
+          for (int t = 0; t < 2; ++t) {
+            const int key0 = j * kBlockN + 32 * t;
+            const _Float16* kp = k0 + (int64_t)min(key0 + ql, keys - 1) * p->ksn;
+            float16v x = (float16v)0.0f;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) x = E::mfma(*(const half8*)(kp + 16 * kk), qr[kk], x);
+            // Bit k of seen: key key0 + 4 hi + k is visible, k = 8 (i / 4) + i % 4 for
+            // element i.
+            const int n = last - key0 - 4 * hi;
+            uint32_t seen = (t == 0 ? (uint32_t)word : (uint32_t)(word >> 32)) >> (4 * hi);
+            if (n < 31) seen &= n < 0 ? 0u : (2u << n) - 1u;
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) {
+              float pr[2];
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                const int32_t keep = (int32_t)(seen << (31 - (8 * (i >> 2) + (i & 3) + e))) >> 31;
+                pr[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i + e], c, -off));
+                pr[e] = __builtin_bit_cast(float, __builtin_bit_cast(int32_t, pr[e]) & keep);
+              }
+              sum = E::sum2(E::pack(pr[0], pr[1]), sum);
+            }
+          }
+        }
+        return sum;
+      };
+      l_run = lacc[0];
+      // (pair mode, a group 1 that moved on: its share of A in the exchange area too)
+      for (int seg = 0; seg < (g1b ? 2 : 1); ++seg) {
+        const bool of_b = g1b && seg == 0;
+        float l = l_run, m = m_run;
+        if constexpr (PAIRS) {
+          if (seg == 1) {
+            l = pair_xo[MT * 1024 + 64 + lane];
+            m = pair_xo[MT * 1024 + lane];
+          }
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(l != l) == 0, 1)) continue;
+        l = sum_again(of_b ? qrow_b : qrow, of_b ? max(tile0, block_tiles) - block_tiles : tile0,
+                      of_b ? tile_end - block_tiles : g1b ? block_tiles : tile_end, m);
+        if constexpr (PAIRS) {
+          if (seg == 1) {
+            pair_xo[MT * 1024 + 64 + lane] = l;
+            continue;
+          }
+        }
+        l_run = l;
+      }
+    }
 
     if constexpr (KSPLIT) {
       // Group 1 wave w+4 hands its O (unnormalised), running max and partial
