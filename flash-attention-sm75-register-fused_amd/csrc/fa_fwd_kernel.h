@@ -1149,26 +1149,30 @@ void launch_fused(const FwdArgs& a, int batch, bool causal, Schedule schedule,
                      stream, args)
   constexpr bool RS = D == 64;
   // Non-causal launches without a mask: by rounds (see ROWSUM), counted in
-  // 128-row blocks for either workgroup shape, and none on the dynamic
-  // schedule, so that the kernels forced for a call give the same bits.
+  // 128-row blocks for either workgroup shape and schedule: the kernels that can
+  // be forced for a call then give the same bits.
   constexpr bool RS_FULL = RS && (MASK != 0 || KSPLIT);
+  bool one_round = false;
   if constexpr (RS && !RS_FULL) {
     FwdArgs planned = a;
-    if (!dyn && !causal && plan_grid(planned, batch, 128) <= slots) {
-      if (same) FA_LAUNCH(false, true, RS, false); else FA_LAUNCH(false, false, RS, false);
-      return;
-    }
+    one_round = !causal && plan_grid(planned, batch, 128) <= slots;
   }
   if constexpr (WAVES == 4) {
     if (dyn) {
       if (causal) {
         if (same) FA_LAUNCH(true, true, RS, true); else FA_LAUNCH(true, false, RS, true);
+      } else if (one_round) {
+        if (same) FA_LAUNCH(false, true, RS, true); else FA_LAUNCH(false, false, RS, true);
       } else {
         if (same) FA_LAUNCH(false, true, RS_FULL, true);
         else FA_LAUNCH(false, false, RS_FULL, true);
       }
       return;
     }
+  }
+  if (one_round) {
+    if (same) FA_LAUNCH(false, true, RS, false); else FA_LAUNCH(false, false, RS, false);
+    return;
   }
   if (causal) {
     if (same) FA_LAUNCH(true, true, RS, false); else FA_LAUNCH(true, false, RS, false);
