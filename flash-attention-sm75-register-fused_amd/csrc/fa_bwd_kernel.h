@@ -990,10 +990,15 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
       step(j, u_c, I1{}, next_c);
     };
     if (ntiles > j_begin) {
-      load_tile(j_begin, I0{});
-      load_tile(j_begin + 1, I1{});  // (zeros past the keys)
+      // The first tile has landed once all but the second's loads have: these are
+      // the only ones after the fence (a plain load, as of the mask word, may move
+      // freely on either side of it, and one that moves past it makes the wait
+      // stricter).
       if (MASK) mw = mrow[j_begin];
-      barrier_after_loads<2 * SEGQ + (MASK ? 1 : 0)>();  // the first tile has landed
+      load_tile(j_begin, I0{});
+      fence_schedule();
+      load_tile(j_begin + 1, I1{});  // (zeros past the keys)
+      barrier_after_loads<2 * SEGQ>();
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
         sb[0] = E::mfma(rd.row(k_lds0, 0, kk), qf[kk], kk == 0 ? (float16v)0.0f : sb[0]);
