@@ -40,7 +40,6 @@
 #include <chrono>
 
 #include "fa_internal.h"
-#include "flash_attn_sm75.h"
 
 #include "fa_kernel_common.h"
 
@@ -986,7 +985,8 @@ constexpr int kDecLongTiles = 64, kDecLongMinTiles = 8;
 constexpr int kSmallMinTiles = 8;
 constexpr int kTargetWgs = 256;  // one workgroup per CU
 
-int plan_splits(const DecodePlan& pl, int head_dim) {
+// (`most`: splits the workspace has room for.)
+int plan_splits(const DecodePlan& pl, int head_dim, int64_t most) {
   const bool blocks = pl.row_blocks > 1;
   const int no_split = blocks ? (head_dim == 64 ? 36 : 27) : head_dim == 64 ? 20 : 12;
   if (pl.tiles <= no_split) return 1;
@@ -997,14 +997,15 @@ int plan_splits(const DecodePlan& pl, int head_dim) {
   if (blocks) {
     if (pl.tiles > kDecLongTiles)  // one block per CU, a long range each: halve it
       splits = std::max(splits, std::min(2, (kTargetWgs + pl.units - 1) / pl.units));
-    else if (head_dim == 64 && splits < 4)
+    else if (head_dim == 64 && std::min<int64_t>(splits, most) < 4)
       splits = 1;
   } else {
     const int two = 2 * kTargetWgs / pl.units;
     if (7 * splits * pl.units < 6 * kTargetWgs && two * pl.units > 9 * splits * pl.units / 4)
       splits = two;
   }
-  return std::max(1, std::min(std::min(splits, kMaxSplits), pl.tiles / min_tiles));
+  splits = std::min(std::min(splits, kMaxSplits), pl.tiles / min_tiles);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(splits, most));
 }
 
 }  // namespace
@@ -1020,30 +1021,21 @@ DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
   int64_t nk_eff = a.nk;
   if (causal) nk_eff = std::min<int64_t>(a.nk, std::max<int64_t>(0, (int64_t)a.n + a.diag));
   pl.tiles = (int)((nk_eff + kDecTile - 1) / kDecTile);
-  const int splits = plan_splits(pl, head_dim);
+  // One split's partials and its mark (merge in the split-K kernel).  A
+  // workspace with room for fewer splits than the GPU wants gets those; one with
+  // room for the partials alone, the combine kernel.
+  const int64_t record = (int64_t)pl.units * pl.rows * (head_dim + 2) * 4;
+  const int64_t mark = (int64_t)pl.units * 8;
+  const int splits = plan_splits(pl, head_dim, workspace_bytes / record);
   pl.chunk_tiles = std::max(1, (pl.tiles + splits - 1) / splits);
   pl.splits = std::max(1, (pl.tiles + pl.chunk_tiles - 1) / pl.chunk_tiles);
   pl.merge_in_kernel = pl.splits > 1 && pl.splits <= kThreads &&
                        (int64_t)pl.splits * pl.rows * head_dim * 4 <= kMergeMaxBytes &&
                        (head_dim != 64 || pl.splits <= kMergeMaxSplits64 ||
-                        (int64_t)pl.units * pl.splits <= kMergeFewWgs);
-  pl.workspace_bytes = 0;
-  if (pl.splits > 1) {
-    // Partials, then the marks in whole records of one split (a size of that
-    // many splits more), or alone where those would not fit the no-allocation
-    // entry's scratch.
-    const int64_t record = (int64_t)pl.units * pl.rows * (head_dim + 2) * 4;
-    const int64_t marks = pl.merge_in_kernel ? (int64_t)pl.units * pl.splits * 8 : 0;
-    pl.workspace_bytes = record * (pl.splits + (marks + record - 1) / record);
-    if (pl.workspace_bytes > (int64_t)FA_SM75_NOALLOC_SCRATCH_BYTES)
-      pl.workspace_bytes = record * pl.splits + marks;
-  }
-  if (pl.workspace_bytes > workspace_bytes) {  // not enough room: one split
-    pl.splits = 1;
-    pl.chunk_tiles = std::max(1, pl.tiles);
-    pl.merge_in_kernel = false;
-    pl.workspace_bytes = 0;
-  }
+                        (int64_t)pl.units * pl.splits <= kMergeFewWgs) &&
+                       pl.splits * (record + mark) <= workspace_bytes;
+  pl.workspace_bytes =
+      pl.splits > 1 ? pl.splits * (record + (pl.merge_in_kernel ? mark : 0)) : 0;
   return pl;
 }
 
