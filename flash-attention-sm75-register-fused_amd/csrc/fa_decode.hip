@@ -102,9 +102,14 @@ constexpr int kMergeMaxBytes = 64 << 10;
 // every CU then ends with a merge of short partials, which the next launch
 // cannot overlap (B=2 Hq=8 Hkv=8 4096 keys d64, 16 units of 16 splits: 9.5
 // merged here, 8.8 by the combine kernel; B=16 H=1 16384 keys 16.9 and 16.1;
-// 8 splits, B=4 H=8 4096 keys, 11.5 and 11.6).
+// 8 splits, B=4 H=8 4096 keys, 11.5 and 11.6).  Row blocks, whose units are
+// many as well, up to 5 splits and 48 KB (8 splits of 32 columns at head_dim 64,
+// 8 heads 128 x 2600 11.3 merged here and 10.2, 6 splits 11.3 and 11.0, 5 11.7
+// and 11.9; head_dim 128, 4 splits, 8 heads 256 x 2600 17.8 and 17.3, 3 24.6
+// and 25.0).
 constexpr int kMergeMaxSplits64 = 8;
 constexpr int kMergeFewWgs = 128;
+constexpr int kMergeMaxBlockBytes = 48 << 10, kMergeMaxBlockSplits = 5;
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -957,21 +962,27 @@ bool decode_eligible(const FwdArgs& a, int batch) {
 
 namespace {
 
-// How many workgroups share a unit's keys.  A workgroup (four waves) streams
-// K and V at about 50 bytes/ns however many loads it has in flight (16 KB per
-// 32-key tile at head_dim 128), so few workgroups are slow and the split
-// spreads a unit over CUs; the merge costs 2-3 us.  Timed on MI355X through
-// the C ABI, bfloat16, us per call:
-//  * few tiles run as one split: decode Hq=14 Hkv=2 d64 512 keys 5.9 against
-//    7.7 for 4 splits, Hq=32 Hkv=8 d128 256 keys 7.1 against 8.7; one head of
-//    1024 rows d64 8.2 against 8.8, two of 777 d128 13.4 against 14.4; and so
-//    do row blocks (32 columns, a longer merge) that could only be halved and
-//    have at most 64 tiles at head_dim 64 (4 heads of 1024 rows 9.6 against
-//    10.3);
-//  * a split has at least kDecMinTiles tiles, one per wave, and at head_dim
-//    64 eight where the range is long (4097 keys 8.7 against 9.0 for 32
-//    splits); row blocks eight (one head of 1024 rows d128 16.1 -> 12.9, 4
-//    heads 300 x 2000 29.6 -> 16.2);
+// How many workgroups share a unit's keys.  A workgroup (four waves, one tile
+// of 32 keys each in flight) streams K and V at about 50 bytes/ns at head_dim
+// 128 (16 KB per tile) and half that at 64, so few workgroups are slow and the
+// split spreads a unit over CUs; the merge costs 1-3 us.  Timed on MI355X,
+// bfloat16, us per call:
+//  * few tiles run as one split: decode at head_dim 128 up to 15 (Hq=32 Hkv=8
+//    385 keys 8.6 against 9.4 for 3 splits, 16 sequences 448 keys 9.4 and 10.4),
+//    at 64 up to 20 (Hq=14 Hkv=2 512 keys 5.9 against 7.7 for 4 splits), 28 for
+//    more than 64 units (8 x 12 heads 704 keys 7.7 and 9.4, 896 keys 8.6 and
+//    9.7; 16 x 8 heads 918 keys 9.2 and 9.3, 1078 keys 10.0 and 9.8); row
+//    blocks (32 columns, a longer merge) up to 36 at head_dim 64 and 28 at 128
+//    (one head of 1024 rows d64 8.2 against 8.8; 8 heads 448 x 896 d128 14.1 and
+//    14.6, 448 x 960 15.7 and 14.8), and at 64 up to 64 where they could only
+//    be halved (4 heads of 1024 rows 9.6 against 10.3);
+//  * a split has at least four tiles, one per wave; at head_dim 64, of fewer than
+//    eight there are at most 16, or 8 where a unit is one row or 16 would not be
+//    merged in the kernel (16 splits against one per eight tiles at 65-125 tiles:
+//    Hq=14 Hkv=2 7.9-8.2 and 8.2-8.5, 4 sequences 8.1-8.3 and 8.3-8.8; 8 splits
+//    against 16 at 44-64 tiles: 2 x 8 heads 8.1-8.4 and 8.9, one head level;
+//    4097 keys 8.4 for 15 splits, 8.7 for 17, 9.0 for 32); row blocks eight
+//    (one head of 1024 rows d128 16.1 -> 12.9, 4 heads 300 x 2000 29.6 -> 16.2);
 //  * the workgroups fill whole rounds of CUs: rounding the split count up
 //    put two workgroups on some CUs and one on others, and the launch took
 //    as long as two (B=3 Hq=32 Hkv=8 9000 keys d128: 264 workgroups 31.7,
@@ -980,22 +991,26 @@ namespace {
 //    workgroups of a CU run together) if that fills them better: the latter
 //    480 workgroups 67.4, B=20 Hq=8 3000 keys d128 160 workgroups 48.2, 480
 //    44.3.
-constexpr int kDecMinTiles = 4;
-constexpr int kDecLongTiles = 64, kDecLongMinTiles = 8;
-constexpr int kSmallMinTiles = 8;
+constexpr int kDecMinTiles = 4, kMinTiles = 8;
+constexpr int kBlockLongTiles = 64;
 constexpr int kTargetWgs = 256;  // one workgroup per CU
 
 // (`most`: splits the workspace has room for.)
 int plan_splits(const DecodePlan& pl, int head_dim, int64_t most) {
   const bool blocks = pl.row_blocks > 1;
-  const int no_split = blocks ? (head_dim == 64 ? 36 : 27) : head_dim == 64 ? 20 : 12;
+  const bool many = 4 * pl.units > kTargetWgs;  // fewer than four splits a unit in one round
+  const int no_split =
+      blocks ? (head_dim == 64 ? 36 : 28) : head_dim == 64 ? (many ? 28 : 20) : 15;
   if (pl.tiles <= no_split) return 1;
-  const int min_tiles = blocks ? kSmallMinTiles
-                        : head_dim == 64 && pl.tiles > kDecLongTiles ? kDecLongMinTiles
-                                                                     : kDecMinTiles;
+  int limit = pl.tiles / (blocks ? kMinTiles : kDecMinTiles);
+  if (!blocks && head_dim == 64) {
+    const bool one_row = pl.rows == 1;
+    const int most_short = one_row || 16 * pl.units > kMergeFewWgs ? 8 : 16;
+    limit = std::max(std::min(limit, most_short), (pl.tiles + (one_row ? 7 : 0)) / kMinTiles);
+  }
   int splits = std::max(1, kTargetWgs / pl.units);
   if (blocks) {
-    if (pl.tiles > kDecLongTiles)  // one block per CU, a long range each: halve it
+    if (pl.tiles > kBlockLongTiles)  // one block per CU, a long range each: halve it
       splits = std::max(splits, std::min(2, (kTargetWgs + pl.units - 1) / pl.units));
     else if (head_dim == 64 && std::min<int64_t>(splits, most) < 4)
       splits = 1;
@@ -1004,7 +1019,7 @@ int plan_splits(const DecodePlan& pl, int head_dim, int64_t most) {
     if (7 * splits * pl.units < 6 * kTargetWgs && two * pl.units > 9 * splits * pl.units / 4)
       splits = two;
   }
-  splits = std::min(std::min(splits, kMaxSplits), pl.tiles / min_tiles);
+  splits = std::min(std::min(splits, kMaxSplits), limit);
   return (int)std::max<int64_t>(1, std::min<int64_t>(splits, most));
 }
 
@@ -1029,11 +1044,16 @@ DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
   const int splits = plan_splits(pl, head_dim, workspace_bytes / record);
   pl.chunk_tiles = std::max(1, (pl.tiles + splits - 1) / splits);
   pl.splits = std::max(1, (pl.tiles + pl.chunk_tiles - 1) / pl.chunk_tiles);
-  pl.merge_in_kernel = pl.splits > 1 && pl.splits <= kThreads &&
-                       (int64_t)pl.splits * pl.rows * head_dim * 4 <= kMergeMaxBytes &&
-                       (head_dim != 64 || pl.splits <= kMergeMaxSplits64 ||
-                        (int64_t)pl.units * pl.splits <= kMergeFewWgs) &&
-                       pl.splits * (record + mark) <= workspace_bytes;
+  const int64_t partial_o = (int64_t)pl.splits * pl.rows * head_dim * 4;
+  pl.merge_in_kernel =
+      pl.splits > 1 && pl.splits <= kThreads && pl.splits * (record + mark) <= workspace_bytes;
+  if (pl.row_blocks > 1)
+    pl.merge_in_kernel = pl.merge_in_kernel && partial_o <= kMergeMaxBlockBytes &&
+                         pl.splits <= kMergeMaxBlockSplits;
+  else
+    pl.merge_in_kernel = pl.merge_in_kernel && partial_o <= kMergeMaxBytes &&
+                         (head_dim != 64 || pl.splits <= kMergeMaxSplits64 ||
+                          (int64_t)pl.units * pl.splits <= kMergeFewWgs);
   pl.workspace_bytes =
       pl.splits > 1 ? pl.splits * (record + (pl.merge_in_kernel ? mark : 0)) : 0;
   return pl;
