@@ -85,12 +85,17 @@ inline Schedule schedule_of_policy(int policy) {
 // N=4096 159 -> 128, B=4 Hq=32 Hkv=8 N=2048 d128 161 -> 131, B=2 N=8192 866 ->
 // 856; backward B=2 Hq=32 Hkv=8 N=4096 d128 1222 -> 1089, B=8 H=8 N=2048 d64
 // 192 -> 177.  At one workgroup per CU or fewer the locality is worth more
-// (forward B=8 H=8 N=512 d64 12.0 against 12.5), and so it is for one sequence,
-// whose heads hold equal work.  Order only: the same bits.
+// (forward B=8 H=8 N=512 d64 12.0 against 12.5), and so it is for rows of fewer
+// than 512 queries, whose blocks read few tiles each (forward N=448: B=8 Hq=64
+// Hkv=8 d128 68.1 against 75.2, B=2 23.1 and 23.9, B=8 Hq=14 Hkv=2 d64 17.2 and
+// 17.9; eleven shapes 0.905-1.011x; N=611 0.90-1.09x, from N=768 mostly above),
+// and for one sequence, whose heads hold equal work.  Order only: the same bits.
+constexpr int kSpreadMinRows = 512;
 template <class Args>
 inline int plan_xcds(const Args& a, int units, int64_t items) {
   const int sequences = units / (a.hq / a.group);
-  const bool uneven = a.mranges != nullptr && a.mrsb != 0 && sequences > 1;
+  const bool uneven =
+      a.mranges != nullptr && a.mrsb != 0 && sequences > 1 && a.n >= kSpreadMinRows;
   if (units % kNumXcds != 0 || (uneven && items > resident_fused_workgroups() / 2)) return 1;
   return kNumXcds;
 }

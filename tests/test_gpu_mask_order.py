@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,N,D", [(4, 8, 2, 1100, 64),   # 288 blocks
                                           (4, 8, 2, 900, 128),   # 256 blocks: unit by unit
                                           (8, 7, 1, 700, 128),   # 336 blocks, a group of 7
-                                          (8, 8, 1, 300, 64)])   # 192 blocks
+                                          (8, 8, 1, 300, 64),    # 192 blocks
+                                          (8, 10, 1, 500, 64)])  # 320 blocks, short rows: unit by unit
 def test_padded_batch_order(device, B, Hq, Hkv, N, D):
     print(f"[mask order] {(B, Hq, Hkv, N, D)}", flush=True)
     g = torch.Generator("cuda").manual_seed(N)
