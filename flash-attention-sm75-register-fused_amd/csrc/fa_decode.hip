@@ -114,6 +114,13 @@ typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
+// The max that a merge of splits takes the others relative to.  Where it is -inf
+// every split so far saw no key, with sum and O zero, or only NaN scores, with
+// both NaN.  Relative to 0 the weight of either is 2^-inf = 0, which leaves the
+// zeros and keeps the NaN (such splits left out, a query with a NaN in it gave
+// zeros where an unsplit call gives NaN).
+__device__ __forceinline__ float finite_max(float m) { return m == -__builtin_inff() ? 0.0f : m; }
+
 // Normalises and stores 4 dimensions of query column c of row block rb of
 // (batch, KV head) bh from the splits' merged max (log2 units), sum and O,
 // and the row's LSE once.  Columns past the last row are not stored.
@@ -609,13 +616,13 @@ __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d)
             if (s0 + u * groups >= d.splits) ml[i][u][0] = -__builtin_inff();
             m_new = fmaxf(m_new, ml[i][u][0]);
           }
-          if (m_new == -__builtin_inff()) continue;
-          const float alpha = __builtin_amdgcn_exp2f(m_acc[i] - m_new);
+          const float m_use = finite_max(m_new);
+          const float alpha = __builtin_amdgcn_exp2f(m_acc[i] - m_use);
           l_acc[i] *= alpha;
           o_acc[i] *= alpha;
 #pragma unroll
           for (int u = 0; u < BATCH; ++u) {
-            const float w = __builtin_amdgcn_exp2f(ml[i][u][0] - m_new);
+            const float w = __builtin_amdgcn_exp2f(ml[i][u][0] - m_use);
             l_acc[i] += w * ml[i][u][1];
             o_acc[i] += w * os[i][u];
           }
@@ -646,12 +653,11 @@ __global__ void __launch_bounds__(kThreads, 2) fa_decode_kernel(const DecArgs d)
     for (int q = 1; q < groups; ++q) Mg = fmaxf(Mg, xm[q * items + tid]);
     float lg = 0.0f;
     v4f og = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (Mg != -__builtin_inff()) {
-      for (int q = 0; q < groups; ++q) {
-        const float w = __builtin_amdgcn_exp2f(xm[q * items + tid] - Mg);
-        lg += w * xm[kThreads + q * items + tid];
-        og += w * __builtin_bit_cast(v4f, xo[q * items + tid]);
-      }
+    const float Mg_use = finite_max(Mg);
+    for (int q = 0; q < groups; ++q) {
+      const float w = __builtin_amdgcn_exp2f(xm[q * items + tid] - Mg_use);
+      lg += w * xm[kThreads + q * items + tid];
+      og += w * __builtin_bit_cast(v4f, xo[q * items + tid]);
     }
     store_merged<D, BF16>(d, bh, rb, tid / (D / 4), 4 * (tid % (D / 4)), Mg, lg, og);
   }
@@ -697,19 +703,18 @@ __global__ void __launch_bounds__(kCombineThreads) fa_decode_combine(const DecAr
   const int grp = tid / D;
   constexpr float kNegInf = -__builtin_inff();
   // Running state of this thread's splits: max (log2 units), sum, O[dim]
-  // relative to that max.  A split that saw no key has max -inf and adds
-  // nothing (2^-inf = 0); while every split so far is such, the state stays
-  // (-inf, 0, 0).
+  // relative to that max (finite_max).  A split that saw no key has max -inf and
+  // adds nothing; while every split so far is such, the state stays (-inf, 0, 0).
   float m_run = kNegInf, l_run = 0.0f, o_run = 0.0f;
   auto fold = [&](int n, const float* ms, const float* ls, const float* os) {
     float m_new = m_run;
     for (int u = 0; u < n; ++u) m_new = fmaxf(m_new, ms[u]);
-    if (m_new == kNegInf) return;
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    const float m_use = finite_max(m_new);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
     l_run *= alpha;
     o_run *= alpha;
     for (int u = 0; u < n; ++u) {
-      const float w = __builtin_amdgcn_exp2f(ms[u] - m_new);
+      const float w = __builtin_amdgcn_exp2f(ms[u] - m_use);
       l_run += w * ls[u];
       o_run += w * os[u];
     }
@@ -743,18 +748,16 @@ __global__ void __launch_bounds__(kCombineThreads) fa_decode_combine(const DecAr
 #pragma unroll
   for (int q = 1; q < GROUPS; ++q) M = fmaxf(M, m_grp[q]);
   float o = 0.0f, Ltot = 0.0f;
-  if (M != kNegInf) {
+  const float m_use = finite_max(M);
 #pragma unroll
-    for (int q = 0; q < GROUPS; ++q) {
-      const float w = __builtin_amdgcn_exp2f(m_grp[q] - M);
-      o += w * o_grp[q][dim];
-      Ltot += w * l_grp[q];
-    }
+  for (int q = 0; q < GROUPS; ++q) {
+    const float w = __builtin_amdgcn_exp2f(m_grp[q] - m_use);
+    o += w * o_grp[q][dim];
+    Ltot += w * l_grp[q];
   }
   const float inv = (Ltot > 0.0f) ? (1.0f / Ltot) : 0.0f;
   a.o[b * a.osb + hq * a.osh + (int64_t)qi * a.osn + dim] = Elem<BF16>::round(o * inv);
   if (a.lse != nullptr && dim == 0) {
-    const float m_use = (M == -__builtin_inff()) ? 0.0f : M;
     a.lse[((int64_t)b * a.hq + hq) * a.n + qi] =
         (m_use + __builtin_log2f(Ltot)) * 0.69314718055994530942f;
   }
@@ -826,15 +829,15 @@ __global__ void __launch_bounds__(kCombineThreads) fa_decode_combine_wide(const 
 #pragma unroll
     for (int u = 0; u < kWideBatch; ++u)
       if (u < n) m_new = fmaxf(m_new, ms[u]);
-    if (m_new == kNegInf) continue;
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    const float m_use = finite_max(m_new);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
     l_run *= alpha;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o_run[e] *= alpha;
 #pragma unroll
     for (int u = 0; u < kWideBatch; ++u) {
       if (u < n) {
-        const float w = __builtin_amdgcn_exp2f(ms[u] - m_new);
+        const float w = __builtin_amdgcn_exp2f(ms[u] - m_use);
         l_run += w * ls[u];
         o_run[0] += w * os[u].x;
         o_run[1] += w * os[u].y;
@@ -855,17 +858,16 @@ __global__ void __launch_bounds__(kCombineThreads) fa_decode_combine_wide(const 
 #pragma unroll
   for (int q = 1; q < kWideGroups; ++q) M = fmaxf(M, m_grp[q]);
   float o[4] = {0.0f, 0.0f, 0.0f, 0.0f}, Ltot = 0.0f;
-  if (M != kNegInf) {
+  const float m_use = finite_max(M);
 #pragma unroll 8
-    for (int q = 0; q < kWideGroups; ++q) {
-      const float w = __builtin_amdgcn_exp2f(m_grp[q] - M);
-      const float4 oq = o_grp[q][lane];
-      o[0] += w * oq.x;
-      o[1] += w * oq.y;
-      o[2] += w * oq.z;
-      o[3] += w * oq.w;
-      Ltot += w * l_grp[q];
-    }
+  for (int q = 0; q < kWideGroups; ++q) {
+    const float w = __builtin_amdgcn_exp2f(m_grp[q] - m_use);
+    const float4 oq = o_grp[q][lane];
+    o[0] += w * oq.x;
+    o[1] += w * oq.y;
+    o[2] += w * oq.z;
+    o[3] += w * oq.w;
+    Ltot += w * l_grp[q];
   }
   const float inv = (Ltot > 0.0f) ? (1.0f / Ltot) : 0.0f;
   half4 v;
@@ -873,7 +875,6 @@ __global__ void __launch_bounds__(kCombineThreads) fa_decode_combine_wide(const 
   for (int e = 0; e < 4; ++e) v[e] = Elem<BF16>::round(o[e] * inv);
   *(half4*)(a.o + b * a.osb + hq * a.osh + (int64_t)qi * a.osn + dim0) = v;
   if (a.lse != nullptr && chunk == 0 && lane == 0) {
-    const float m_use = (M == kNegInf) ? 0.0f : M;
     a.lse[((int64_t)b * a.hq + hq) * a.n + qi] =
         (m_use + __builtin_log2f(Ltot)) * 0.69314718055994530942f;
   }
