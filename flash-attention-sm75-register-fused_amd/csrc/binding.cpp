@@ -363,8 +363,11 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_backward
     const auto bytes = Q.options().dtype(torch::kUInt8);
     try {
       work = torch::empty({ws}, bytes);
-    } catch (const c10::OutOfMemoryError&) {  // the required part alone: no dK/dV split
-      ws = p.batch * p.heads_q * ((p.seq_len + 63) / 64) * 520;
+    } catch (const c10::OutOfMemoryError&) {
+      // The required part alone: no dK/dV split (the split adds up to 134 MB to a
+      // call, and one that ran without them has to go on running).  dK and dV are
+      // then the unsplit sums, whose bits differ.
+      ws = p.batch * p.heads_q * ((p.seq_len + 63) / 64) * FA_SM75_BWD_WORKSPACE_PER_TILE;
       work = torch::empty({ws}, bytes);
     }
     p.workspace = work.data_ptr();

@@ -339,6 +339,10 @@ int validate_bwd(const fa_bwd_params* p) {
   return FA_OK;
 }
 
+static_assert(fa::bwd_workspace_bytes(1, 1, fa::kBwdStatsTile) == FA_SM75_BWD_WORKSPACE_PER_TILE &&
+                  fa::kBwdStatsTile == 64,
+              "the header's required bytes");
+
 // Offset of the dK/dV split's partials in the backward's workspace.
 int64_t bwd_part_offset(const fa_bwd_params* p) {
   return (fa::bwd_workspace_bytes(p->batch, p->heads_q, p->seq_len) + 255) / 256 * 256;

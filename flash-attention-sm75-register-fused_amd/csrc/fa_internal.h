@@ -269,11 +269,11 @@ int64_t plan_bwd_split(const BwdArgs& a, int batch, int head_dim, bool causal, B
 // Workspace bytes a backward call requires: the statistics records, then the
 // query tiles' key spans (BwdArgs::stats, tspans).  The split's partials
 // follow at the next multiple of 256 bytes when the workspace has room.
-inline int64_t bwd_stats_bytes(int64_t batch, int64_t heads_q, int64_t seq_len) {
+constexpr int64_t bwd_stats_bytes(int64_t batch, int64_t heads_q, int64_t seq_len) {
   return batch * heads_q * ((seq_len + kBwdStatsTile - 1) / kBwdStatsTile) *
          (2 * kBwdStatsTile) * (int64_t)sizeof(float);
 }
-inline int64_t bwd_workspace_bytes(int64_t batch, int64_t heads_q, int64_t seq_len) {
+constexpr int64_t bwd_workspace_bytes(int64_t batch, int64_t heads_q, int64_t seq_len) {
   return bwd_stats_bytes(batch, heads_q, seq_len) +
          batch * heads_q * ((seq_len + kBwdStatsTile - 1) / kBwdStatsTile) * 2 *
              (int64_t)sizeof(int32_t);

@@ -287,8 +287,9 @@ typedef struct fa_bwd_params {
   int causal;           /* an fa_causal value (the forward's) */
   int dtype;            /* an fa_dtype */
   void* stream;         /* hipStream_t; NULL selects the default stream */
-  void* workspace;      /* device scratch, 16-byte aligned: 520 bytes per
-                           (batch, query head, 64 query rows) are required,
+  void* workspace;      /* device scratch, 16-byte aligned:
+                           FA_SM75_BWD_WORKSPACE_PER_TILE bytes per (batch,
+                           query head, 64 query rows) are required,
                            fa_sm75_backward_workspace_size() are used; calls
                            that share one race */
   int64_t workspace_bytes;
@@ -314,14 +315,19 @@ void fa_sm75_set_contiguous_bwd_strides(fa_bwd_params* p);
  * argument before touching the device.  Returns FA_OK or an fa_status. */
 int fa_sm75_backward(const fa_bwd_params* p);
 
-/* Workspace bytes fa_sm75_backward uses: 520 per (batch, query head, 64
- * query rows) -- that tile's row statistics, then its span of visible keys
- * when mask_ranges is given -- which are required, and, where one dK/dV
- * workgroup per 128 keys would leave CUs idle, room (at most 134 MB) for the
- * fp32 partials of several per 128 keys.  With less than that the call runs
- * with one.  From the sizes, head_dim and causal flag alone (0 if a size is
- * negative or p is NULL; the required bytes if they are not a valid call's).
- * The same call with the same workspace size gives the same bits. */
+/* Required workspace bytes of fa_sm75_backward per (batch, query head, 64
+ * query rows, the last ones rounded up): the row statistics, then the span of
+ * visible keys when mask_ranges is given. */
+#define FA_SM75_BWD_WORKSPACE_PER_TILE 520
+
+/* Workspace bytes fa_sm75_backward uses: the required ones, and, where one
+ * dK/dV workgroup per 128 keys would leave CUs idle, room for the fp32 partials
+ * of several per 128 keys (at most four pieces per CU: 134 MB at head_dim 128 on
+ * 256 CUs).  With less than that the call runs with one.  From the sizes,
+ * head_dim, the causal flag, whether mask_bits is set and the current device,
+ * which has to be the call's (0 if a size is negative or p is NULL; the required
+ * bytes if they are not a valid call's).  The same call with the same workspace
+ * size gives the same bits. */
 int64_t fa_sm75_backward_workspace_size(const fa_bwd_params* p);
 
 #define FA_SM75_ABI_VERSION 7
