@@ -1063,8 +1063,10 @@ __global__ void __launch_bounds__(256, MASK && D == 128 ? 1 : 2) fa_bwd_dq_kerne
           // (bf16, left-padded causal masks: B=4 Hq=16 Hkv=4 N=2048 230 us ->
           // 206, B=2 Hq=32 Hkv=8 N=4096 660 -> 587).  The MASK-free instances
           // meet few such tiles and run 2% slower in this order.
-          // The word's halves are shifted apart: a 64-bit shift by a lane's
-          // amount misreads an amount in the last of 256 registers.
+          // The word's halves are shifted apart: an instance that shifted all
+          // 64 bits by a lane's amount, which sat in the last of its 256
+          // registers, used P of hidden keys now and then.  Why was not shown
+          // (a 64-bit shift reads its amount as a register pair).
 #pragma unroll
           for (int i = 0; i < 16; ++i)
             sa[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i], c2, -lse2));

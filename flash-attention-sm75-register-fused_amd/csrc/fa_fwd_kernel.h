@@ -624,8 +624,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) fa_fwd_kernel(const FwdArgs a) 
       if (MASK) need_mask = need_mask || __builtin_amdgcn_ballot_w64(~mw != 0) != 0;
       if (need_mask) {
         // Bit 8 (i / 4) + i % 4 of mws[t]: element (t, i).  The halves are shifted
-        // apart: a 64-bit shift by a lane's amount misreads an amount in the
-        // last of 256 registers.
+        // apart, as in the dQ kernel (fa_bwd_kernel.h).
         const uint32_t mws[2] = {(uint32_t)mw >> (4 * hi), (uint32_t)(mw >> 32) >> (4 * hi)};
         // Element (t, i) holds key kstart + 4 hi + off, off = 32 t + 8 (i / 4)
         // + i % 4 (a constant); it is visible iff off <= lim.

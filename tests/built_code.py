@@ -28,9 +28,10 @@ def _code_object(path):
     vgprs = {}
     for kernel in re.split(r"\n  - (?=\.)", notes)[1:]:
         name = re.search(r"\n    \.name:\s+(\S+)", kernel)
-        count = re.search(r"\.vgpr_count:\s+(\d+)", kernel)
+        # (accumulation registers share the allocation, after the others)
+        count, acc = (re.search(rf"\.{c}_count:\s+(\d+)", kernel) for c in ("vgpr", "agpr"))
         if name and count:
-            vgprs[name.group(1)] = int(count.group(1))
+            vgprs[name.group(1)] = int(count.group(1)) - (int(acc.group(1)) if acc else 0)
     found = []
     for part in re.split(r"\n(?=[0-9a-f]+ <_ZN2fa\S+>:)", asm)[1:]:
         name = re.match(r"[0-9a-f]+ <(\S+)>:", part).group(1)
@@ -42,7 +43,8 @@ def _code_object(path):
 
 
 def kernels():
-    """(mangled name, vector registers, instructions) of every kernel of the library."""
+    """(mangled name, vector registers without accumulation ones, instructions) of every
+    kernel of the library."""
     if not os.path.exists(LIB):
         pytest.fail(f"{LIB} not built: run __graft_entry__.build()")
     if not os.path.exists(os.path.join(LLVM, "llvm-objdump")):
