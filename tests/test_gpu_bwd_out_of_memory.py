@@ -22,6 +22,11 @@ def test_partials_that_do_not_fit(device, causal):
     want = flash_attention_backward(do, q, k, v, o, lse, causal=causal)
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    hogs, held = [], torch.cuda.memory_reserved(device)
+    while torch.cuda.memory_reserved(device) == held:  # no free block takes the partials
+        hogs.append(torch.empty(16 * MB, dtype=torch.uint8, device=device))
+    del hogs[-1]
+    torch.cuda.empty_cache()
     ooms = torch.cuda.memory_stats(device)["num_ooms"]
     total = torch.cuda.get_device_properties(device).total_memory
     # Room for the three gradients in the allocator's 20 MB segments, one or two.
