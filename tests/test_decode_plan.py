@@ -5,11 +5,13 @@ import ctypes
 import os
 
 import pytest
+import test_gpu_split_merge
+import test_gpu_split_nonfinite
 
 from capi_types import LIB, Params
 
 
-def size(B, Hq, Hkv, Nq, Nk, D):
+def size(B, Hq, Hkv, Nq, Nk, D, causal=0):
     if not os.path.exists(LIB):
         pytest.fail(f"{LIB} not built: run __graft_entry__.build()")
     lib = ctypes.CDLL(LIB)
@@ -18,7 +20,7 @@ def size(B, Hq, Hkv, Nq, Nk, D):
     p.q = p.k = p.v = p.o = 0x10000
     p.batch, p.heads_q, p.heads_kv, p.seq_len, p.seq_len_kv, p.head_dim = B, Hq, Hkv, Nq, Nk, D
     lib.fa_sm75_set_contiguous_strides(ctypes.byref(p))
-    p.scale = 0.125
+    p.scale, p.causal = 0.125, causal
     return lib.fa_sm75_workspace_size(ctypes.byref(p))
 
 
@@ -42,3 +44,20 @@ def test_no_cliff_in_the_range(B, Hq, Hkv, Nq, D):
     assert all(sizes[first:])
     # Equal splits of whole tiles: one tile more can take a fifth of them.
     assert all(b >= 0.75 * a for a, b in zip(sizes[first:], sizes[first + 1:]))
+
+
+def merged_by(B, Hq, Hkv, Nq, Nk, D, causal=0):
+    """"kernel" (a mark per workgroup in the workspace), "combine", or None: one split."""
+    s = size(B, Hq, Hkv, Nq, Nk, D, causal)
+    rows = Hq // Hkv * Nq
+    units = B * Hkv * ((rows + 31) // 32)
+    record = units * min(rows, 32) * (D + 2) * 4
+    assert s % record == 0 or s % (record + 8 * units) == 0
+    return None if s == 0 else "combine" if s % record == 0 else "kernel"
+
+
+def test_the_merge_tests_take_the_routes_they_name():
+    K, C = "kernel", "combine"
+    assert [merged_by(*c[:7]) for c in test_gpu_split_merge.CASES] == (
+        [K] * 7 + [None, K, C, C, K, K])
+    assert [merged_by(*c) for c in test_gpu_split_nonfinite.CASES] == [K] * 4 + [C] * 5 + [None]

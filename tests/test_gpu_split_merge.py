@@ -26,8 +26,10 @@ CASES = [
     (2, 8, 2, 3, 700, 64, 2, False),     # bottom-right
     (1, 4, 4, 4, 1500, 128, 1, False),   # top-left, 4 keys seen: one split, then many keys unseen
     (3, 14, 2, 1, 3000, 64, 0, True),    # key bytes: splits that see no key
-    (1, 2, 2, 300, 1100, 128, 2, False), # 32-row blocks, the last one ragged
+    (1, 2, 2, 300, 1100, 128, 2, False), # row blocks merged by the combine kernel
     (1, 1, 1, 200, 2048, 64, 0, False),
+    (1, 4, 4, 777, 1100, 128, 0, False), # row blocks merged here, the last one ragged
+    (1, 2, 2, 1000, 1500, 64, 2, False),
 ]
 
 

@@ -15,8 +15,10 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # B, Hq, Hkv, Nq, Nk, D
     (1, 14, 2, 1, 4097, 64),     # in the kernel, groups of splits
-    (1, 8, 2, 4, 3000, 128),     # in the kernel
-    (1, 2, 2, 200, 1900, 64),    # row blocks, several items per thread
+    (2, 8, 1, 1, 2000, 128),     # in the kernel, one item per thread
+    (1, 9, 1, 1, 1100, 128),     # in the kernel, some threads with two
+    (1, 4, 4, 777, 1100, 128),   # in the kernel, row blocks: four each
+    (1, 2, 2, 200, 1900, 64),    # row blocks, combine
     (2, 8, 8, 1, 4096, 64),      # combine
     (1, 32, 8, 8, 2048, 128),    # combine
     (1, 1, 1, 1, 65536, 64),     # wide combine
