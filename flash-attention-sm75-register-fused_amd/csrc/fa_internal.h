@@ -184,7 +184,7 @@ struct DecodePlan {
   int64_t workspace_bytes;  // 0 when splits == 1
 };
 bool decode_eligible(const FwdArgs& a, int batch);
-// Splits for a workspace of `workspace_bytes` (one split if it is too small).
+// Splits for a workspace of `workspace_bytes`: as many as it has room for, down to one.
 DecodePlan plan_decode(const FwdArgs& a, int batch, int head_dim, bool causal,
                        int64_t workspace_bytes);
 int launch_decode_forward(const FwdArgs& a, const DecodePlan& plan, int head_dim, bool causal,
